@@ -40,6 +40,10 @@ int hk_gemm_xwt(hk_ctx* ctx, int dtype, int n, int out, int in, const void* x, l
 int hk_gemm_xwt_cd(hk_ctx* ctx, int dtype, int cd_dtype, int n, int out, int in, const void* x, long ldx,
                    const void* w, long ldw, void* y, long ldy, const void* c, long ldc, float alpha, float beta);
 
+// Two projections of the same x rows, Y = X W^T and Y2 = X W2^T (contiguous weights and outputs).
+int hk_gemm_xwt_pair(hk_ctx* ctx, int dtype, int n, int in, const void* x, long ldx, int out, const void* w, void* y,
+                     int out2, const void* w2, void* y2);
+
 // hk_qk_norm_rope_kv_write with an optional per-token (sequence, position) table (int pairs,
 // hk_launch_token_seq_pos), which replaces the kernel's search of cu_seqlens
 int hk_qk_norm_rope_kv_write_impl(hk_ctx* ctx, int dtype, const void* q_in, long q_in_tok, long q_in_head,

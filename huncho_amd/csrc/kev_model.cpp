@@ -463,8 +463,7 @@ int kev_forward_impl(hk_kev_model* m, const int32_t* ids, const int32_t* cu_dev,
         RUN(norm_x(m, b.x, L.in_norm, n, b.h));
         if (L.type == 0) {
             const int rows = m->gdn_rows;
-            RUN(hk_gemm_xwt(ctx, dt, n, rows, H, b.h, H, L.w_in, H, b.big, rows, nullptr, 0, 1.0f, 0.0f));
-            RUN(hk_gemm_xwt(ctx, dt, n, m->ba_rows, H, b.h, H, L.w_ba, H, b.ba, m->ba_rows, nullptr, 0, 1.0f, 0.0f));
+            RUN(hk_gemm_xwt_pair(ctx, dt, n, H, b.h, H, rows, L.w_in, b.big, m->ba_rows, L.w_ba, b.ba));
             const int b_col = 0, a_col = Hv;
             const int dk = c.lin_key_dim, dv = c.lin_v_dim;
             if (dt != HK_F32 && c.conv_k == 4 && rows % 8 == 0 && dk == 128 && dv == 128) {
@@ -601,7 +600,7 @@ extern "C" int hk_kev_model_identity(hk_kev_model* m, char* buf, size_t len, siz
          {"recurrent_state_dtype", "fp32"},
          {"causal_conv_execution", f32 || !gdn_mfma || c.conv_k != 4 ? "rocm-gdn-prep-v1" : "rocm-fused-gdn-layer-v1"},
          {"mlp_gate_execution", m->mlp_fused ? "rocm-gemm-swiglu-epilogue-v1" : "rocm-swiglu-v1"},
-         {"projection_kernel", "hipblaslt-pinned-or-heuristic-v1"},
+         {"projection_kernel", f32 ? "hipblaslt-pinned-or-heuristic-v1" : "rocm-gemm-ksplit-few-rows-or-hipblaslt-v1"},
          {"pointer_head_dtype", "fp32"},
          {"library", hk_version()}},
         buf, len, needed);

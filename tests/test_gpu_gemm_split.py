@@ -1,0 +1,70 @@
+"""The few-row GEMM (gemm_split.hip) against a float64 product of the same 16-bit values, through
+hk_linear and through the models' projections, at the edges of its tiles: one row, a row more and
+less than each tile's 32, 64 and 96 rows, K of one to many steps (fewer steps than waves leave a wave
+without any), column counts that leave a part of a tile.
+
+Gates: 1 unit in the last place of the dtype (2^-7 relative for bf16, 2^-10 for fp16) plus the fp32
+accumulation's absolute error over K products; the SwiGLU epilogue 2 units, from the rounded gate
+and up products."""
+import pytest
+import torch
+
+from huncho_amd import abi
+
+pytestmark = pytest.mark.gpu
+
+EPS = {torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from huncho_amd.ops import context_for_torch
+
+    c = context_for_torch(0)
+    yield c
+    c.close()
+
+
+def linear(ctx, x, w, epi=0, c=None, out_cols=None):
+    y = torch.full((x.shape[0] + 1, out_cols or w.shape[0]), 7.0, dtype=x.dtype, device=x.device)
+    dt = abi.HK_BF16 if x.dtype == torch.bfloat16 else abi.HK_F16
+    ctx.check(abi.lib().hk_linear(ctx.h, dt, epi, x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), x.shape[0],
+                                  w.shape[0], x.shape[1], c.data_ptr() if c is not None else None,
+                                  c.stride(0) if c is not None else 0, y.data_ptr(), y.stride(0)))
+    assert bool((y[-1] == 7.0).all())  # nothing is stored past the last row
+    return y[:-1]
+
+
+def within(got, want, dtype, ulps, k):
+    g, w = got.double(), want.double()
+    return bool(((g - w).abs() <= w.abs() * EPS[dtype] * ulps + 4e-7 * k).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [1, 31, 33, 64, 65, 97, 169, 300, 700])
+@pytest.mark.parametrize("n,k", [(256, 64), (1024, 192), (768, 1152), (3584, 320)])
+def test_linear_few_rows(ctx, dtype, rows, n, k):
+    g = torch.Generator(device="cuda").manual_seed(rows * 7 + n + k)
+    pad = torch.randn((rows, k + 8), generator=g, device="cuda").to(dtype) * 0.5
+    x = pad[:, :k]  # a row stride wider than the row
+    w = (torch.randn((n, k), generator=g, device="cuda") * 0.05).to(dtype)
+    ref = x.double() @ w.double().T
+    assert within(linear(ctx, x, w), ref.to(dtype), dtype, 1, k)
+    c = torch.randn((rows, n), generator=g, device="cuda").to(dtype)
+    assert within(linear(ctx, x, w, 1, c), (ref + c.double()).to(dtype), dtype, 1, k)
+    b = ref.view(rows, n // 32, 2, 16).to(dtype).double()
+    gate, up = b[:, :, 0].reshape(rows, -1), b[:, :, 1].reshape(rows, -1)
+    # a gate or up product next to a rounding boundary may round the other way: one unit of each
+    tol = 2 * EPS[dtype] * (gate.abs() * up.abs() + (torch.nn.functional.silu(gate) * up).abs()) + 4e-7 * k
+    got = linear(ctx, x, w, 2, out_cols=n // 2).double()
+    assert bool(((got - torch.nn.functional.silu(gate) * up).abs() <= tol).all())
+
+
+def test_rows_do_not_depend_on_the_batch(ctx):
+    """K is split the same way for every tile, so a row's result is the same bits at any row count."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn((600, 1024), generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn((1024, 1024), generator=g, device="cuda") * 0.05).to(torch.bfloat16)
+    whole = linear(ctx, x, w)
+    for rows in (1, 40, 100, 200, 400):
+        assert torch.equal(linear(ctx, x[:rows], w), whole[:rows])
