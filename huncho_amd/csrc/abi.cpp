@@ -86,6 +86,11 @@ extern "C" int hk_ctx_destroy(hk_ctx* ctx) {
     hipStreamSynchronize(ctx->stream);
     hk_noalloc_scratch_release(ctx);
     hk_blas_release(ctx);
+    if (ctx->gdn_scratch) {
+        hipDeviceSynchronize();  // its users may be on streams that the context has left
+        hipFree(ctx->gdn_scratch);
+    }
+    if (ctx->gdn_moved) hipEventDestroy(ctx->gdn_moved);
     if (ctx->fault_dev) hipFree(ctx->fault_dev);
     if (ctx->own_stream) hipStreamDestroy(ctx->own_stream);
     delete ctx;
@@ -94,8 +99,63 @@ extern "C" int hk_ctx_destroy(hk_ctx* ctx) {
 
 extern "C" int hk_ctx_set_stream(hk_ctx* ctx, void* hip_stream) {
     if (!ctx) return HK_ERR_INVALID;
-    ctx->stream = (hipStream_t)hip_stream;  // NULL is HIP's null stream
+    const hipStream_t next = (hipStream_t)hip_stream;  // NULL is HIP's null stream
+    if (next != ctx->stream && ctx->gdn_scratch_used) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        const bool ok = hipStreamIsCapturing(ctx->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone &&
+                        (ctx->gdn_moved || hipEventCreateWithFlags(&ctx->gdn_moved, hipEventDisableTiming) == hipSuccess) &&
+                        hipEventRecord(ctx->gdn_moved, ctx->stream) == hipSuccess;
+        (void)hipGetLastError();
+        ctx->gdn_wait = true;
+        ctx->gdn_wait_all = !ok;
+        ctx->gdn_scratch_used = false;
+    }
+    ctx->stream = next;
     return HK_OK;
+}
+
+size_t hk_gdn_split_bytes(int n_tokens, int n_seqs, int heads) {
+    return (size_t)(n_tokens / 64 + n_seqs) * heads * hk::HK_GDN_SPLIT_SLOT;
+}
+
+bool hk_gdn_scratch_reserve(hk_ctx* ctx, size_t bytes) {
+    if (bytes <= ctx->gdn_scratch_bytes) return true;
+    if (bytes > kGdnScratchMax) return false;
+    size_t size = 32u << 20;
+    while (size < bytes) size <<= 1;
+    bytes = size;
+    if (ctx->gdn_scratch) {
+        hipDeviceSynchronize();
+        hipFree(ctx->gdn_scratch);
+        ctx->gdn_scratch = nullptr;
+        ctx->gdn_scratch_bytes = 0;
+        ctx->gdn_scratch_used = ctx->gdn_wait = ctx->gdn_wait_all = false;
+    }
+    if (hipMalloc(&ctx->gdn_scratch, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        ctx->gdn_scratch = nullptr;
+        return false;
+    }
+    ctx->gdn_scratch_bytes = bytes;
+    return true;
+}
+
+// The scratch for a call on the context's stream, after the users on other streams, or null: too small
+// (grown only if may_alloc) or the stream is being captured (a graph may be replayed on any stream).
+static void* gdn_scratch_for(hk_ctx* ctx, size_t bytes, bool may_alloc) {
+    if (bytes > (may_alloc ? kGdnScratchMax : ctx->gdn_scratch_bytes)) return nullptr;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (!hk_gdn_scratch_reserve(ctx, bytes)) return nullptr;
+    if (ctx->gdn_wait) {
+        if (ctx->gdn_wait_all || hipStreamWaitEvent(ctx->stream, ctx->gdn_moved, 0) != hipSuccess) hipDeviceSynchronize();
+        ctx->gdn_wait = ctx->gdn_wait_all = false;
+    }
+    ctx->gdn_scratch_used = true;
+    return ctx->gdn_scratch;
 }
 
 extern "C" void* hk_ctx_own_stream(hk_ctx* ctx) { return ctx ? (void*)ctx->own_stream : nullptr; }
@@ -584,13 +644,23 @@ extern "C" int hk_swiglu(hk_ctx* ctx, int dtype, const void* gu, long gu_tok, lo
 
 // The fused layer with optional per-sequence row tables for the state and the conv history
 // (device arrays of n_seqs pointers; used by the cached model forward).
+// Whether the batch takes the three-kernel form of the fused layer (gdn16_split.hip): few chains (pairs of
+// a row and a head), whose rows are several chunks long on average. Measured, 16 heads, bf16, us, one
+// kernel against three, by rows x tokens:
+//   1 x 128 26.7 21.8, x 512 95.8 28.5, x 2048 386 66.6, x 4096 767 117;  4 x 128 26.7 23.6, x 512 99.3
+//   45.3, x 2048 384 165;  6 x 128 26.8 29.4, x 256 50.3 42.8;  8 x 128 26.7 32.1, x 256 52.0 46.9, x 1024 197 161
+static bool gdn_split_takes(int n_seqs, int n_tokens, int heads) {
+    const long chains = (long)n_seqs * heads, chunks = n_tokens / 64;
+    return chains <= 64 ? chunks >= 2L * n_seqs : chains <= 128 && chunks >= 4L * n_seqs;
+}
+
 int hk_gdn_fused_rows(hk_ctx* ctx, int dtype, const void* mixed, long mixed_tok, const float* conv_w, int conv_k,
                       const void* conv_hist, void* conv_tail_out, const void* ba, long ba_tok, int b_col, int a_col,
                       const float* base_g, const float* dt_bias, const void* z, long z_tok, const float* norm_w,
                       float eps, const int32_t* cu, int n_seqs, int n_tokens, int heads, int k_heads,
                       const float* initial_state, float* final_state, void* out, long out_tok,
                       const float* const* init_rows, float* const* final_rows, const void* const* hist_rows,
-                      void* const* tail_rows) {
+                      void* const* tail_rows, bool may_alloc) {
     if (!ctx) return HK_ERR_INVALID;
     if (dtype != HK_BF16 && dtype != HK_F16)
         return hk_fail(ctx, HK_ERR_UNSUPPORTED, "fused Gated DeltaNet layer: 16-bit dtypes only (got %d)", dtype);
@@ -617,6 +687,12 @@ int hk_gdn_fused_rows(hk_ctx* ctx, int dtype, const void* mixed, long mixed_tok,
                   final_state, out, out_tok, heads, n_tokens, ctx->fault_dev, init_rows, final_rows};
     hk::GdnFusedArgs fa{mixed, mixed_tok, conv_w, (int)conv_dim, conv_hist, conv_tail_out, ba, ba_tok, b_col, a_col,
                         base_g, dt_bias, 1.0f / sqrtf(128.0f), k_heads, z, z_tok, norm_w, eps, hist_rows, tail_rows};
+    if (gdn_split_takes(n_seqs, n_tokens, heads)) {
+        if (void* scratch = gdn_scratch_for(ctx, hk_gdn_split_bytes(n_tokens, n_seqs, heads), may_alloc)) {
+            const int rc = hk_launch_gdn16_split(dtype, &a, &fa, n_seqs, n_tokens / 64 + n_seqs, scratch, ctx->stream);
+            return rc ? hk_fail(ctx, rc, "fused Gated DeltaNet launch failed") : HK_OK;
+        }
+    }
     int rc = hk_launch_gdn16(dtype, 1, &a, &fa, n_seqs, ctx->stream);
     return rc ? hk_fail(ctx, rc, "fused Gated DeltaNet launch failed") : HK_OK;
 }
@@ -628,7 +704,7 @@ extern "C" int hk_gdn_fused(hk_ctx* ctx, int dtype, const void* mixed, long mixe
                             int k_heads, const float* initial_state, float* final_state, void* out, long out_tok) {
     return hk_gdn_fused_rows(ctx, dtype, mixed, mixed_tok, conv_w, conv_k, conv_hist, conv_tail_out, ba, ba_tok, b_col,
                              a_col, base_g, dt_bias, z, z_tok, norm_w, eps, cu, n_seqs, n_tokens, heads, k_heads,
-                             initial_state, final_state, out, out_tok, nullptr, nullptr, nullptr, nullptr);
+                             initial_state, final_state, out, out_tok, nullptr, nullptr, nullptr, nullptr, true);
 }
 
 // ---------------------------------------------------------------------------

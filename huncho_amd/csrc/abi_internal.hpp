@@ -20,7 +20,21 @@ struct hk_ctx {
     int* fault_dev = nullptr;
     std::string last_error;
     hk_blas* blas = nullptr;
+    // Scratch of the fused Gated DeltaNet layer for few, long rows: at most kGdnScratchMax bytes, kept
+    // until the context is destroyed. Work on it is ordered by the stream; when the context moves to
+    // another stream, gdn_moved marks the end of the old stream's use and the next use waits for it.
+    void* gdn_scratch = nullptr;
+    size_t gdn_scratch_bytes = 0;
+    bool gdn_scratch_used = false;     // on the current stream, since the last move
+    hipEvent_t gdn_moved = nullptr;
+    bool gdn_wait = false, gdn_wait_all = false;
 };
+constexpr size_t kGdnScratchMax = 512u << 20;
+// Ensures `bytes` of scratch (rounded up to a power of two, at least 32 MiB); frees and reallocates a smaller one after waiting
+// for its users. false if bytes exceed the limit or the allocation fails.
+bool hk_gdn_scratch_reserve(hk_ctx* ctx, size_t bytes);
+// Bytes for the chunks of n_tokens tokens in n_seqs rows.
+size_t hk_gdn_split_bytes(int n_tokens, int n_seqs, int heads);
 
 int hk_fail(hk_ctx* ctx, int code, const char* fmt, ...);
 int hk_check_hip(hk_ctx* ctx, hipError_t e, const char* what);

@@ -139,9 +139,7 @@ __device__ __forceinline__ float wave_incl_scan(float x, int lane) {
 // In place, the inverses T_bb = (I + A_bb)^-1 of the four 16x16 diagonal blocks of the
 // strictly lower A [64][AS], by forward substitution on waves 0-3 (wave w: block w, lane j:
 // column j). The strictly lower part of each solved block keeps its zeros above the diagonal.
-// Kept out of line: inlined, its unrolled row loads would be hoisted together and spill the
-// caller.
-static __device__ __attribute__((noinline)) void solve_diagonal_blocks(float* Am, int wave, int lane) {
+__device__ __forceinline__ void solve_diagonal_blocks_inline(float* Am, int wave, int lane) {
     if (wave >= 4) return;
     const int b = wave * 16, j = lane & 15;
     float x[16];
@@ -165,6 +163,12 @@ static __device__ __attribute__((noinline)) void solve_diagonal_blocks(float* Am
 #pragma unroll
         for (int i = 0; i < 16; ++i) Am[(b + i) * AS + b + j] = x[i];
     }
+}
+
+// The same out of line for gdn_chunk16: inlined there, its unrolled row loads would be hoisted together
+// and spill the caller.
+static __device__ __attribute__((noinline)) void solve_diagonal_blocks(float* Am, int wave, int lane) {
+    solve_diagonal_blocks_inline(Am, wave, lane);
 }
 
 // Two runs of four 16-bit elements of a Q / K row: columns x0 .. x0 + 3 and x0 + 16 .. + 19
@@ -204,6 +208,228 @@ __device__ __forceinline__ typename M16<T>::v4 ld_a4(const float* Am, int r, int
     const f32x4 x = *(const f32x4*)(Am + r * AS + c);
     return NEG ? typename M16<T>::v4{(T)-x[0], (T)-x[1], (T)-x[2], (T)-x[3]}
                : typename M16<T>::v4{(T)x[0], (T)x[1], (T)x[2], (T)x[3]};
+}
+
+// P0 of the fused layer: the conv, SiLU and l2norm of chunk rows c0 .. c0 + 63 of q, k and v (the raw
+// in_proj rows of the sequence that starts at token t0) into the LDS tiles.
+template <typename T>
+__device__ __forceinline__ void fused_rows(const GdnFusedArgs& fa, int t0, int Tn, int c0, int h, int kh, const T* hist,
+                                           int wave, int q4, int j, f16* Qs, f16* Ks, f16* Vs) {
+    typedef f16 CT;
+    typedef typename M16<CT>::v8 v8;
+    typedef typename M16<T>::v8 tv8;
+    typedef typename M16<T>::v2 tv2;
+    // 16 lane groups (4 per wave) x 4 rows of each of q, k and v: group G = 4 wave + q4
+    // takes chunk rows 4 G .. 4 G + 3 of every tensor, so all four waves share the conv,
+    // SiLU and l2norm evenly. Each tensor's 4 conv outputs come from a 7-row window of raw
+    // conv inputs (sequence positions c0 + 4 G - 3 ..). Positions past the sequence end
+    // are loaded clamped: they only reach rows past the end, whose beta is 0 and whose
+    // outputs are not stored. Positions before the start are the conv history or 0.
+    const int r0 = 4 * (4 * wave + q4);
+    auto tcol = [&](int tsr) {  // mixed column of this lane's channels in tensor tsr
+        return (tsr == 2 ? 2 * (long)fa.Hk * 128 + (long)h * 128 : (long)tsr * fa.Hk * 128 + (long)kh * 128) +
+               8 * j;
+    };
+    // all three windows are loaded before the first conv, so the chunk waits for one
+    // memory round trip
+    // Addresses: a wave-uniform base per tensor (this sequence's first row, the head's
+    // columns) plus one 32-bit byte offset per row shared by the three tensors (the host
+    // keeps n_tokens * mixed_tok * sizeof(T) below 2^32 and the row stride below 2^24)
+    tv8 raw[3][7];
+    {
+        const char* const mb = (const char*)fa.mixed + (long)t0 * fa.mixed_tok * (long)sizeof(T);
+        const char* const base[3] = {mb + (long)kh * 128 * sizeof(T),
+                                     mb + ((long)fa.Hk + kh) * 128 * sizeof(T),
+                                     mb + (2L * fa.Hk + h) * 128 * sizeof(T)};
+        const unsigned row_b = (unsigned)(fa.mixed_tok * sizeof(T));
+#pragma unroll
+        for (int i = 0; i < 7; ++i) {
+            const int p = c0 + r0 - 3 + i;
+            const unsigned pc = (unsigned)(p < 0 ? 0 : (p >= Tn ? Tn - 1 : p));
+            const unsigned off = __umul24(pc, row_b) + 16u * j;
+#pragma unroll
+            for (int tsr = 0; tsr < 3; ++tsr) raw[tsr][i] = *(const tv8*)(base[tsr] + off);
+        }
+    }
+    if (c0 + r0 == 0) {  // windows start 3 positions before the sequence
+#pragma unroll
+        for (int tsr = 0; tsr < 3; ++tsr) {
+            if (hist) {
+                const T* hb = hist + tcol(tsr) * 3;
+#pragma unroll
+                for (int i = 0; i < 3; ++i)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) raw[tsr][i][e] = hb[e * 3 + i];
+            } else {
+#pragma unroll
+                for (int i = 0; i < 3; ++i) raw[tsr][i] = tv8{};
+            }
+        }
+    }
+#pragma unroll
+    for (int tsr = 0; tsr < 3; ++tsr) {
+        const long mct = tcol(tsr);
+        CT* dst = tsr == 0 ? Qs : tsr == 1 ? Ks : Vs;
+        // taps (0, 1) and (2, 3) of each channel as 16-bit pairs (the weights are the
+        // model dtype's values, exact in T)
+        tv2 w01[8], w23[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const f32x4 w4 = *(const f32x4*)(fa.conv_w + (mct + e) * 4);
+            w01[e] = tv2{(T)w4[0], (T)w4[1]};
+            w23[e] = tv2{(T)w4[2], (T)w4[3]};
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float y[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float acc = dot2(w23[e], tv2{raw[tsr][i + 2][e], raw[tsr][i + 3][e]},
+                                       dot2_0(w01[e], tv2{raw[tsr][i][e], raw[tsr][i + 1][e]}));
+                y[e] = silu(acc);
+            }
+            // the conv output is stored in T (qwen3_5.rs:843), held exactly in CT
+            f16x2 o[4];
+            if (tsr < 2) {  // conv output stored in the activation dtype, then l2norm over
+                            // the head's 128 channels (16 lanes); q also takes the scale
+                tv2 p[4];
+#pragma unroll
+                for (int m = 0; m < 4; ++m) p[m] = tv2{(T)y[2 * m], (T)y[2 * m + 1]};
+                float ss = dot2_0(p[0], p[0]);
+#pragma unroll
+                for (int m = 1; m < 4; ++m) ss = dot2(p[m], p[m], ss);
+                ss = sum16(ss);
+                const float inv = fast_rsqrt(ss + 1e-6f) * (tsr == 0 ? fa.scale : 1.0f);
+                // the normalised q and k stay fp32 in the reference (l2norm returns
+                // fp32, qwen3_5.rs:204-210, 923-924): rounded only to the fp16 operand
+#pragma unroll
+                for (int m = 0; m < 4; ++m) o[m] = f16x2{(f16)(lo_f(p[m]) * inv), (f16)(hi_f(p[m]) * inv)};
+            } else {
+#pragma unroll
+                for (int m = 0; m < 4; ++m) o[m] = rnd_ct<T>(y[2 * m], y[2 * m + 1]);
+            }
+            *(v8*)(dst + el(r0 + i, 8 * j)) = __builtin_bit_cast(v8, o);
+        }
+    }
+}
+
+// P1's tiles of A = strict_lower(beta e^(G_t - G_s) k_t.k_s) in fp32 and Aqk = lower(e^(G_t - G_s) q_t.k_s).
+__device__ __forceinline__ void chunk_tiles(const f16* Qs, const f16* Ks, const float* Gs, const float* Bs, float* Am,
+                                            f16* Aq, int wave, int q4, int j) {
+    typedef f16 CT;
+    typedef typename M16<CT>::v8 v8;
+    typedef typename M16<CT>::v4 v4;
+    // lower tile pairs p = (ti, si), si <= ti: wave w takes pairs w, w + 4, w + 8; upper tiles
+    // (0,1) (0,2) (0,3) (1,2) (1,3) (2,3) of A and Aqk are zeroed, wave w taking w and w + 4.
+    // The products are formed transposed (K_s as the A operand): lane (q4, j) holds keys
+    // s = 16 si + 4 q4 + r of query / key row t = 16 ti + j, four consecutive columns of
+    // row t of A and Aqk, written as one vector each.
+    for (int p = wave; p < 10; p += 4) {
+        const int ti = p < 1 ? 0 : p < 3 ? 1 : p < 6 ? 2 : 3;
+        const int si = p - (ti * (ti + 1)) / 2;
+        f32x4 kk = f32x4{0.f, 0.f, 0.f, 0.f}, qk = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            const v8 ka = *(const v8*)(Ks + el(16 * si + j, 32 * ks + 8 * q4));
+            kk = M16<CT>::mma(ka, *(const v8*)(Ks + el(16 * ti + j, 32 * ks + 8 * q4)), kk);
+            qk = M16<CT>::mma(ka, *(const v8*)(Qs + el(16 * ti + j, 32 * ks + 8 * q4)), qk);
+        }
+        const int t = 16 * ti + j, s4 = 16 * si + 4 * q4;
+        const float gt = Gs[t], bt = Bs[t];
+        const f32x4 gs = *(const f32x4*)(Gs + s4);
+        f32x4 av, qv;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int s = s4 + r;
+            // exp(G_t - G_s) may overflow above the diagonal; the selects drop it there
+            const float ex = __expf(gt - gs[r]);
+            const float dec = s <= t ? ex : 0.0f;
+            av[r] = s < t ? bt * dec * kk[r] : 0.0f;
+            qv[r] = dec * qk[r];
+        }
+        *(f32x4*)(Am + t * AS + s4) = av;
+        *(v4*)(Aq + t * TS + s4) = pack1<CT>(qv);
+    }
+    for (int u = wave; u < 6; u += 4) {
+        const int ti = u < 3 ? 0 : u < 5 ? 1 : 2;
+        const int si = u < 3 ? u + 1 : u < 5 ? u - 1 : 3;
+        const int t = 16 * ti + j, s4 = 16 * si + 4 * q4;
+        *(f32x4*)(Am + t * AS + s4) = f32x4{0.f, 0.f, 0.f, 0.f};
+        *(v4*)(Aq + t * TS + s4) = v4{};
+    }
+}
+
+// beta = sigmoid(b) and g = -exp(A_log) softplus(a + dt_bias) of token tt
+template <typename T>
+__device__ __forceinline__ void fused_g_beta(const GdnFusedArgs& fa, long tt, int h, float& gv, float& bv) {
+    const T* row = (const T*)fa.ba + tt * fa.ba_tok;
+    const float b = f(row[fa.b_col + h]);
+    const float av = f(row[fa.a_col + h]);
+    bv = rnd<T>(fast_sigmoid(b));
+    gv = fa.base_g[h] * __logf(__expf(av + fa.dt_bias[h]) + 1.0f);
+}
+
+// The gate norm_w * silu(z) of a thread's four output rows 16 pass + rrow, columns 8 rsub .. + 7 (rows
+// past the end read a clamped row and are not stored)
+template <typename T>
+__device__ __forceinline__ void gate_rows(const GdnFusedArgs& fa, int t0, int c0, int Lc, int h, int rsub, int rrow,
+                                          float (&gz)[4][8]) {
+    typedef typename M16<T>::v8 tv8;
+    tv8 zv[4];
+    const char* const zb = (const char*)fa.z + ((long)t0 * fa.z_tok + (long)h * DV) * (long)sizeof(T);
+#pragma unroll
+    for (int pass = 0; pass < 4; ++pass) {
+        const unsigned tt = (unsigned)(c0 + min(pass * 16 + rrow, Lc - 1));
+        zv[pass] = *(const tv8*)(zb + (__umul24(tt, (unsigned)(fa.z_tok * sizeof(T))) + 16u * rsub));
+    }
+#pragma unroll
+    for (int pass = 0; pass < 4; ++pass)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) gz[pass][e] = fa.norm_w[8 * rsub + e] * silu(f(zv[pass][e]));
+}
+
+// One row of the gated RMSNorm: rms(o) * gz, stored if `in` at row t of the sequence (ob: its first row,
+// this head). True if the row is not finite: a 16-bit operand out of fp16 range.
+template <typename T>
+__device__ __forceinline__ bool store_gated(const GdnFusedArgs& fa, long o_tok, char* ob, f16x8 ov, const float (&gz)[8],
+                                            int t, bool in, int rsub) {
+    typedef typename M16<T>::v8 tv8;
+    float x[8], ss = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        x[e] = f(ov[e]);
+        ss += x[e] * x[e];
+    }
+    ss = sum16(ss);
+    const float inv = fast_rsqrt(ss * (1.0f / 128.0f) + fa.eps);
+    tv8 y;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) y[e] = (T)((x[e] * inv) * gz[e]);
+    if (in) *(tv8*)(ob + (__umul24((unsigned)t, (unsigned)(o_tok * sizeof(T))) + 16u * rsub)) = y;
+    return in && !(ss < __builtin_inff());
+}
+
+// The cache tail: the last 3 raw conv inputs of [history, sequence] of the 8 channels at mixed column mc
+template <typename T>
+__device__ __forceinline__ void write_tail(const GdnFusedArgs& fa, int t0, int Tn, long mc, const T* hist, T* tail) {
+    typedef typename M16<T>::v8 tv8;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const int p = Tn - 3 + i;
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = 0.0f;
+        if (p >= 0) {
+            tv8 x = *(const tv8*)((const T*)fa.mixed + (long)(t0 + p) * fa.mixed_tok + mc);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = f(x[e]);
+        } else if (hist) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = f(hist[((long)mc + e) * 3 + (p + 3)]);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) tail[((long)mc + e) * 3 + i] = (T)v[e];
+    }
 }
 
 template <typename T, bool FUSED>
@@ -284,98 +510,7 @@ __global__ __launch_bounds__(256, 2) void gdn_chunk16(GdnArgs a, GdnFusedArgs fa
         __syncthreads();
         // ---------------- P0: inputs -> LDS ----------------
         if (FUSED) {
-            // 16 lane groups (4 per wave) x 4 rows of each of q, k and v: group G = 4 wave + q4
-            // takes chunk rows 4 G .. 4 G + 3 of every tensor, so all four waves share the conv,
-            // SiLU and l2norm evenly. Each tensor's 4 conv outputs come from a 7-row window of raw
-            // conv inputs (sequence positions c0 + 4 G - 3 ..). Positions past the sequence end
-            // are loaded clamped: they only reach rows past the end, whose beta is 0 and whose
-            // outputs are not stored. Positions before the start are the conv history or 0.
-            const int r0 = 4 * (4 * wave + q4);
-            auto tcol = [&](int tsr) {  // mixed column of this lane's channels in tensor tsr
-                return (tsr == 2 ? 2 * (long)fa.Hk * 128 + (long)h * 128 : (long)tsr * fa.Hk * 128 + (long)kh * 128) +
-                       8 * j;
-            };
-            // all three windows are loaded before the first conv, so the chunk waits for one
-            // memory round trip
-            // Addresses: a wave-uniform base per tensor (this sequence's first row, the head's
-            // columns) plus one 32-bit byte offset per row shared by the three tensors (the host
-            // keeps n_tokens * mixed_tok * sizeof(T) below 2^32 and the row stride below 2^24)
-            tv8 raw[3][7];
-            {
-                const char* const mb = (const char*)fa.mixed + (long)t0 * fa.mixed_tok * (long)sizeof(T);
-                const char* const base[3] = {mb + (long)kh * 128 * sizeof(T),
-                                             mb + ((long)fa.Hk + kh) * 128 * sizeof(T),
-                                             mb + (2L * fa.Hk + h) * 128 * sizeof(T)};
-                const unsigned row_b = (unsigned)(fa.mixed_tok * sizeof(T));
-#pragma unroll
-                for (int i = 0; i < 7; ++i) {
-                    const int p = c0 + r0 - 3 + i;
-                    const unsigned pc = (unsigned)(p < 0 ? 0 : (p >= Tn ? Tn - 1 : p));
-                    const unsigned off = __umul24(pc, row_b) + 16u * j;
-#pragma unroll
-                    for (int tsr = 0; tsr < 3; ++tsr) raw[tsr][i] = *(const tv8*)(base[tsr] + off);
-                }
-            }
-            if (c0 + r0 == 0) {  // windows start 3 positions before the sequence
-#pragma unroll
-                for (int tsr = 0; tsr < 3; ++tsr) {
-                    if (hist) {
-                        const T* hb = hist + tcol(tsr) * 3;
-#pragma unroll
-                        for (int i = 0; i < 3; ++i)
-#pragma unroll
-                            for (int e = 0; e < 8; ++e) raw[tsr][i][e] = hb[e * 3 + i];
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < 3; ++i) raw[tsr][i] = tv8{};
-                    }
-                }
-            }
-#pragma unroll
-            for (int tsr = 0; tsr < 3; ++tsr) {
-                const long mct = tcol(tsr);
-                CT* dst = tsr == 0 ? Qs : tsr == 1 ? Ks : Vs;
-                // taps (0, 1) and (2, 3) of each channel as 16-bit pairs (the weights are the
-                // model dtype's values, exact in T)
-                tv2 w01[8], w23[8];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const f32x4 w4 = *(const f32x4*)(fa.conv_w + (mct + e) * 4);
-                    w01[e] = tv2{(T)w4[0], (T)w4[1]};
-                    w23[e] = tv2{(T)w4[2], (T)w4[3]};
-                }
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    float y[8];
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const float acc = dot2(w23[e], tv2{raw[tsr][i + 2][e], raw[tsr][i + 3][e]},
-                                               dot2_0(w01[e], tv2{raw[tsr][i][e], raw[tsr][i + 1][e]}));
-                        y[e] = silu(acc);
-                    }
-                    // the conv output is stored in T (qwen3_5.rs:843), held exactly in CT
-                    f16x2 o[4];
-                    if (tsr < 2) {  // conv output stored in the activation dtype, then l2norm over
-                                    // the head's 128 channels (16 lanes); q also takes the scale
-                        tv2 p[4];
-#pragma unroll
-                        for (int m = 0; m < 4; ++m) p[m] = tv2{(T)y[2 * m], (T)y[2 * m + 1]};
-                        float ss = dot2_0(p[0], p[0]);
-#pragma unroll
-                        for (int m = 1; m < 4; ++m) ss = dot2(p[m], p[m], ss);
-                        ss = sum16(ss);
-                        const float inv = fast_rsqrt(ss + 1e-6f) * (tsr == 0 ? fa.scale : 1.0f);
-                        // the normalised q and k stay fp32 in the reference (l2norm returns
-                        // fp32, qwen3_5.rs:204-210, 923-924): rounded only to the fp16 operand
-#pragma unroll
-                        for (int m = 0; m < 4; ++m) o[m] = f16x2{(f16)(lo_f(p[m]) * inv), (f16)(hi_f(p[m]) * inv)};
-                    } else {
-#pragma unroll
-                        for (int m = 0; m < 4; ++m) o[m] = rnd_ct<T>(y[2 * m], y[2 * m + 1]);
-                    }
-                    *(v8*)(dst + el(r0 + i, 8 * j)) = __builtin_bit_cast(v8, o);
-                }
-            }
+            fused_rows<T>(fa, t0, Tn, c0, h, kh, hist, wave, q4, j, Qs, Ks, Vs);
         } else {
             // 3 tensors x 64 rows x 16 chunks = 12 chunks per lane; 16 lanes per row
             tv8 x[12];
@@ -403,11 +538,7 @@ __global__ __launch_bounds__(256, 2) void gdn_chunk16(GdnArgs a, GdnFusedArgs fa
             if (lane < Lc) {
                 const long tt = t0 + c0 + lane;
                 if (FUSED) {
-                    const T* row = (const T*)fa.ba + tt * fa.ba_tok;
-                    const float b = f(row[fa.b_col + h]);
-                    const float av = f(row[fa.a_col + h]);
-                    bv = rnd<T>(fast_sigmoid(b));
-                    gv = fa.base_g[h] * __logf(__expf(av + fa.dt_bias[h]) + 1.0f);
+                    fused_g_beta<T>(fa, tt, h, gv, bv);
                 } else {
                     gv = a.g[tt * a.gb_tok + h];
                     bv = a.beta[tt * a.gb_tok + h];
@@ -418,44 +549,7 @@ __global__ __launch_bounds__(256, 2) void gdn_chunk16(GdnArgs a, GdnFusedArgs fa
         }
         __syncthreads();
         // ---------------- P1: A, Aqk tiles; K S0, Q S0 ----------------
-        // lower tile pairs p = (ti, si), si <= ti: wave w takes pairs w, w + 4, w + 8; upper tiles
-        // (0,1) (0,2) (0,3) (1,2) (1,3) (2,3) of A and Aqk are zeroed, wave w taking w and w + 4.
-        // The products are formed transposed (K_s as the A operand): lane (q4, j) holds keys
-        // s = 16 si + 4 q4 + r of query / key row t = 16 ti + j, four consecutive columns of
-        // row t of A and Aqk, written as one vector each.
-        for (int p = wave; p < 10; p += 4) {
-            const int ti = p < 1 ? 0 : p < 3 ? 1 : p < 6 ? 2 : 3;
-            const int si = p - (ti * (ti + 1)) / 2;
-            f32x4 kk = f32x4{0.f, 0.f, 0.f, 0.f}, qk = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {
-                const v8 ka = *(const v8*)(Ks + el(16 * si + j, 32 * ks + 8 * q4));
-                kk = M16<CT>::mma(ka, *(const v8*)(Ks + el(16 * ti + j, 32 * ks + 8 * q4)), kk);
-                qk = M16<CT>::mma(ka, *(const v8*)(Qs + el(16 * ti + j, 32 * ks + 8 * q4)), qk);
-            }
-            const int t = 16 * ti + j, s4 = 16 * si + 4 * q4;
-            const float gt = Gs[t], bt = Bs[t];
-            const f32x4 gs = *(const f32x4*)(Gs + s4);
-            f32x4 av, qv;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int s = s4 + r;
-                // exp(G_t - G_s) may overflow above the diagonal; the selects drop it there
-                const float ex = __expf(gt - gs[r]);
-                const float dec = s <= t ? ex : 0.0f;
-                av[r] = s < t ? bt * dec * kk[r] : 0.0f;
-                qv[r] = dec * qk[r];
-            }
-            *(f32x4*)(Am + t * AS + s4) = av;
-            *(v4*)(Aq + t * TS + s4) = pack1<CT>(qv);
-        }
-        for (int u = wave; u < 6; u += 4) {
-            const int ti = u < 3 ? 0 : u < 5 ? 1 : 2;
-            const int si = u < 3 ? u + 1 : u < 5 ? u - 1 : 3;
-            const int t = 16 * ti + j, s4 = 16 * si + 4 * q4;
-            *(f32x4*)(Am + t * AS + s4) = f32x4{0.f, 0.f, 0.f, 0.f};
-            *(v4*)(Aq + t * TS + s4) = v4{};
-        }
+        chunk_tiles(Qs, Ks, Gs, Bs, Am, Aq, wave, q4, j);
         // per token tile tt and column tile cw: R = beta (V - e^G K S0) and, transposed (lane
         // (q4, j): value columns 16 cw + 4 q4 + r of token 16 tt + j), Og = e^G Q S0
         f32x4 R[2][4], Og[2][4];
@@ -588,17 +682,7 @@ __global__ __launch_bounds__(256, 2) void gdn_chunk16(GdnArgs a, GdnFusedArgs fa
         const int rsub = tid & 15, rrow = tid >> 4;  // 16 lanes per row, 16 rows per pass
         float gz[4][8];
         if (FUSED) {
-            tv8 zv[4];
-            const char* const zb = (const char*)fa.z + ((long)t0 * fa.z_tok + (long)h * DV) * (long)sizeof(T);
-#pragma unroll
-            for (int pass = 0; pass < 4; ++pass) {
-                const unsigned tt = (unsigned)(c0 + min(pass * 16 + rrow, Lc - 1));
-                zv[pass] = *(const tv8*)(zb + (__umul24(tt, (unsigned)(fa.z_tok * sizeof(T))) + 16u * rsub));
-            }
-#pragma unroll
-            for (int pass = 0; pass < 4; ++pass)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) gz[pass][e] = fa.norm_w[8 * rsub + e] * silu(f(zv[pass][e]));
+            gate_rows<T>(fa, t0, c0, Lc, h, rsub, rrow, gz);
         }
         __syncthreads();
         // ---------------- P4: O -> HBM (gated RMSNorm when fused) ----------------
@@ -609,20 +693,7 @@ __global__ __launch_bounds__(256, 2) void gdn_chunk16(GdnArgs a, GdnFusedArgs fa
             const v8 ov = *(const v8*)(Os + el(r, 8 * rsub));
             const long tt = t0 + c0 + r;
             if (FUSED) {
-                float x[8], ss = 0.0f;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    x[e] = f(ov[e]);
-                    ss += x[e] * x[e];
-                }
-                ss = sum16(ss);
-                // a 16-bit operand out of fp16 range makes the row non-finite
-                if (r < Lc && !(ss < __builtin_inff())) range_bad = true;
-                const float inv = fast_rsqrt(ss * (1.0f / 128.0f) + fa.eps);
-                tv8 y;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) y[e] = (T)((x[e] * inv) * gz[pass][e]);
-                if (r < Lc) *(tv8*)(ob + (__umul24((unsigned)(c0 + r), (unsigned)(a.o_tok * sizeof(T))) + 16u * rsub)) = y;
+                if (store_gated<T>(fa, a.o_tok, ob, ov, gz[pass], c0 + r, r < Lc, rsub)) range_bad = true;
             } else if (r < Lc) {
                 tv8 y;
                 float ss = 0.0f;
@@ -648,28 +719,7 @@ __global__ __launch_bounds__(256, 2) void gdn_chunk16(GdnArgs a, GdnFusedArgs fa
 #pragma unroll
                 for (int r = 0; r < 4; ++r) sp[(16 * rb + r) * DV + 16 * cw] = S[cw][rb][r];
     }
-    const long mc = mcol + 8 * (ln & 15);
-    if (FUSED && tail && wave < 3 && (ln >> 4) == 0) {
-        // cache tail: the last 3 raw conv inputs of [history, sequence]; wave ts writes the
-        // channels of q, k or v (16 lanes x 8 channels)
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            const int p = Tn - 3 + i;
-            float v[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = 0.0f;
-            if (p >= 0) {
-                tv8 x = *(const tv8*)((const T*)fa.mixed + (long)(t0 + p) * fa.mixed_tok + mc);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) v[e] = f(x[e]);
-            } else if (hist) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) v[e] = f(hist[((long)mc + e) * 3 + (p + 3)]);
-            }
-#pragma unroll
-            for (int e = 0; e < 8; ++e) tail[((long)mc + e) * 3 + i] = (T)v[e];
-        }
-    }
+    if (FUSED && tail && wave < 3 && (ln >> 4) == 0) write_tail<T>(fa, t0, Tn, mcol + 8 * (ln & 15), hist, tail);
 }
 
 }  // namespace gdn16

@@ -75,6 +75,9 @@ struct GdnFusedArgs {
     void* const* tail_rows;
 };
 
+// Scratch bytes of one (64-token chunk, head) of the fused layer for few, long rows (gdn16_split.hip)
+constexpr int HK_GDN_SPLIT_SLOT = 114688;
+
 struct KvArgs {
     const void* q_in;
     long q_in_tok, q_in_head;
@@ -332,6 +335,8 @@ int hk_launch_seq_lens(const int* cu, int n, int* out, hipStream_t st);
 int hk_launch_token_seq_pos(const int* cu, const int* ctxl, int n_seqs, int n_tokens, int* out, int* fault,
                             hipStream_t st);
 int hk_launch_readout(int dtype, const hk::ReadoutArgs* a, hipStream_t st);
+int hk_launch_gdn16_split(int dtype16, const hk::GdnArgs* a, const hk::GdnFusedArgs* fa, int n_seqs, int n_slots,
+                          void* scratch, hipStream_t stream);
 int hk_launch_gemm(int dtype16, int epi, const hk::GemmArgs* a, hipStream_t stream);
 float hk_gemm_split_cost(int epi, const hk::GemmArgs* a);
 int hk_launch_gemm_split(int dtype16, int epi, const hk::GemmArgs* a, hipStream_t stream);

@@ -84,4 +84,4 @@ int hk_gdn_fused_rows(hk_ctx* ctx, int dtype, const void* mixed, long mixed_tok,
                       float eps, const int32_t* cu, int n_seqs, int n_tokens, int heads, int k_heads,
                       const float* initial_state, float* final_state, void* out, long out_tok,
                       const float* const* init_rows, float* const* final_rows, const void* const* hist_rows,
-                      void* const* tail_rows);
+                      void* const* tail_rows, bool may_alloc);

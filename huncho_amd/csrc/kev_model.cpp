@@ -229,6 +229,12 @@ extern "C" int hk_kev_model_create(hk_ctx* ctx, int dtype, const hk_kev_config* 
         hk_rope_fill_table(c.rotary_dim, c.rope_theta, c.max_context, dtype, cs.data(), sn.data());
         if ((rc = upload_f32(m, cs, &m->rope_cos)) || (rc = upload_f32(m, sn, &m->rope_sin))) return fail(rc);
     }
+    // scratch for up to four rows of max_context tokens through the Gated DeltaNet layers, at most half
+    // of the limit, so that no forward allocates (batches that do not fit run the layer without it)
+    if (dtype != HK_F32 && c.conv_k == 4 && c.lin_key_dim == 128 && c.lin_v_dim == 128) {
+        const size_t want = hk_gdn_split_bytes(4 * (c.max_context < 65536 ? c.max_context : 65536), 4, c.lin_n_v_heads);
+        hk_gdn_scratch_reserve(ctx, want < kGdnScratchMax / 2 ? want : kGdnScratchMax / 2);
+    }
     hipStreamSynchronize(nullptr);  // the weight copies, on the null stream, are complete before the
                                     // context's stream (non-blocking) uses them
     *out = m;
@@ -472,7 +478,8 @@ int kev_forward_impl(hk_kev_model* m, const int32_t* ids, const int32_t* cu_dev,
                                       a_col, L.base_g, L.dt_bias, (char*)b.big + (size_t)m->conv_dim * e, rows, L.norm_w,
                                       c.eps, cu_dev, n_seqs, n, Hv, Hk, nullptr, nullptr, b.o, (long)Hv * dv,
                                       view ? view->init_rows[gi] : nullptr, view ? view->final_rows[gi] : nullptr,
-                                      view ? view->hist_rows[gi] : nullptr, view ? view->tail_rows[gi] : nullptr));
+                                      view ? view->hist_rows[gi] : nullptr, view ? view->tail_rows[gi] : nullptr,
+                                      false));
             } else {
                 // the cache's per-sequence conv tails and states, as in the fused path
                 RUN(hk_gdn_prep_rows(ctx, dt, b.big, rows, L.conv_w, c.conv_k, nullptr, b.ba, m->ba_rows, b_col, a_col,
