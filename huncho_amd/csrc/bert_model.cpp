@@ -336,7 +336,7 @@ extern "C" int hk_bert_model_identity(hk_bert_model* m, char* buf, size_t len, s
                                                       : f32        ? "rocm-varlen-bidir-f32-v1"
                                                                    : "rocm-varlen-bidir-mfma-16bit-v1"},
                               {"padding", "unpadded-varlen-v1"},
-                              {"projection_kernel", f32 ? "hipblaslt-pinned-or-heuristic-v1" : "rocm-gemm-ksplit-few-rows-or-hipblaslt-v1"},
+                              {"projection_kernel", f32 ? "hipblaslt-pinned-or-heuristic-v1" : "rocm-gemm-few-rows-or-hipblaslt-v1"},
                               {"library", hk_version()}},
                              buf, len, needed);
 }

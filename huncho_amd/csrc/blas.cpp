@@ -206,7 +206,7 @@ int hk_gemm_xwt(hk_ctx* ctx, int dtype, int n, int out, int in, const void* x, l
 
 // The few-row kernel takes this product: 16-bit operands, whole K steps, 16-byte aligned rows and
 // strides within its 32-bit copy offsets.
-static bool split_takes(int dtype, int epi, const hk::GemmArgs& a) {
+static bool few_rows_takes(int dtype, int epi, const hk::GemmArgs& a) {
     if (dtype != HK_BF16 && dtype != HK_F16) return false;
     const long ldc = a.c ? a.ldc : 0;
     if (a.K <= 0 || a.K % 64 || a.N <= 0 || a.N % (epi == hk::EPI_SWIGLU ? 32 : 8) || a.N2 % 8 || a.ldx % 8 || a.ldw % 8 ||
@@ -215,19 +215,23 @@ static bool split_takes(int dtype, int epi, const hk::GemmArgs& a) {
     return (((uintptr_t)a.x | (uintptr_t)a.w | (uintptr_t)a.c | (uintptr_t)a.y | (uintptr_t)a.w2 | (uintptr_t)a.y2) & 15) == 0;
 }
 
-// A model's projection takes the few-row kernel while its tiles cost no more than about two rounds of
-// them. Beside the library's choice (kernel times, bf16, us): 8192 x 1024 at 169 rows (cost 5.3) 10.1
-// against 13.6, at 300 rows (10.6) 16.2 against 15.2; 6144 x 1024 at 300 rows (8.8) 11.9 against 16.5;
-// 1024 x 3584 + residual at 1200 rows (5.3) 19.5 against 25.3, at 2704 (10.6) 49 against 36; 2304 x
-// 768 at 600 rows (7.0) 9.1 against 10.9; 768 x 1152 + residual at 600 rows (3.1) 5.8 against 10.2.
-static const float kSplitLimit = 10.0f;
+// A model's projection takes the few-row kernel where its estimated time (us) is no more than about the
+// library's. Kernel times beside the library's choice, bf16: 8192 x 1024 at 169 rows 9.5 against 13.6, at
+// 450 rows 15.5 against 16.5, at 600 rows 22.9 against 17.3 (library); 6144 x 1024 at 600 rows 15.6 against
+// 19.2; 1024 x 3584 + residual at 300 rows 13.5 against 14.7, at 1700 rows 25.5 against 29, at 2704 rows
+// 38.7 against 36 (library); 2304 x 768 at 1200 rows 10.0 against 17.1. Both give the same bits.
+static bool few_rows_wins(int epi, const hk::GemmArgs& a) {
+    const float k = (float)a.K / 1024.0f;
+    const float lib = 5.0f + 2.2f * k + 0.9f * 2e-9f * (float)a.M * (float)(a.N + a.N2) * (float)a.K;
+    return 2.2f + k * hk_gemm_few_rows_cost(epi, &a) <= 1.1f * lib;
+}
 
 int hk_gemm_xwt_pair(hk_ctx* ctx, int dtype, int n, int in, const void* x, long ldx, int out, const void* w, void* y,
                      int out2, const void* w2, void* y2) {
     const hk::GemmArgs a{x, w, nullptr, y, ldx, in, 0, out, n, out, in, w2, y2, out2, out2};
-    if (n > 0 && ctx->blas && !ctx->blas->autotune && split_takes(dtype, hk::EPI_STORE, a) &&
-        hk_gemm_split_cost(hk::EPI_STORE, &a) <= kSplitLimit)
-        return hk_launch_gemm_split(dtype, hk::EPI_STORE, &a, ctx->stream) ? hk_fail(ctx, HK_ERR_DEVICE, "gemm launch failed")
+    if (n > 0 && ctx->blas && !ctx->blas->autotune && few_rows_takes(dtype, hk::EPI_STORE, a) &&
+        few_rows_wins(hk::EPI_STORE, a))
+        return hk_launch_gemm_few_rows(dtype, hk::EPI_STORE, &a, ctx->stream) ? hk_fail(ctx, HK_ERR_DEVICE, "gemm launch failed")
                                                                            : HK_OK;
     if (int rc = hk_gemm_xwt(ctx, dtype, n, out, in, x, ldx, w, in, y, out, nullptr, 0, 1.0f, 0.0f)) return rc;
     return hk_gemm_xwt(ctx, dtype, n, out2, in, x, ldx, w2, in, y2, out2, nullptr, 0, 1.0f, 0.0f);
@@ -242,8 +246,8 @@ int hk_gemm_xwt_cd(hk_ctx* ctx, int dtype, int cd_dtype, int n, int out, int in,
     if (!B->autotune && alpha == 1.0f && (!has_c || beta == 1.0f) && (cd_dtype == dtype || (has_c && cd_dtype == HK_F32))) {
         const int epi = !has_c ? hk::EPI_STORE : cd_dtype == dtype ? hk::EPI_RESIDUAL : hk::EPI_RESIDUAL_F32;
         const hk::GemmArgs a{x, w, has_c ? c : nullptr, y, ldx, ldw, has_c ? ldc : 0, ldy, n, out, in, nullptr, nullptr, 0, 0};
-        if (split_takes(dtype, epi, a) && hk_gemm_split_cost(epi, &a) <= kSplitLimit)
-            return hk_launch_gemm_split(dtype, epi, &a, ctx->stream) ? hk_fail(ctx, HK_ERR_DEVICE, "gemm launch failed")
+        if (few_rows_takes(dtype, epi, a) && few_rows_wins(epi, a))
+            return hk_launch_gemm_few_rows(dtype, epi, &a, ctx->stream) ? hk_fail(ctx, HK_ERR_DEVICE, "gemm launch failed")
                                                                      : HK_OK;
     }
     if (!has_c) {
@@ -390,10 +394,10 @@ int hk_gemm_native(hk_ctx* ctx, int dtype, int epi, int n, int out, int in, cons
     hk::GemmArgs a{x, w, epi == hk::EPI_RESIDUAL ? c : nullptr, y, ldx, ldw, ldc, ldy, n, out, in, nullptr, nullptr, 0, 0};
     // The 256 x 256 tiles of gemm.hip cost about 30 K / 1024 us per round of 256 workgroups, however few
     // the rows; the few-row kernel's tiles less while there are few of them (7168 x 1024 SwiGLU at 600
-    // rows 23 against 34 us, at 1200 rows 36.5 against 35.5; 1024 x 3584 at 2704 rows 42 against 99).
+    // rows 21 against 34 us, at 1700 rows 39 against 35; 1024 x 3584 at 2704 rows 38.7 against 99).
     const int tiles = out / 256 * ((n + 255) / 256);
-    if (split_takes(dtype, epi, a) && hk_gemm_split_cost(epi, &a) < 30.0f * (float)((tiles + 255) / 256))
-        return hk_launch_gemm_split(dtype, epi, &a, ctx->stream) ? hk_fail(ctx, HK_ERR_DEVICE, "gemm launch failed") : HK_OK;
+    if (few_rows_takes(dtype, epi, a) && hk_gemm_few_rows_cost(epi, &a) < 30.0f * (float)((tiles + 255) / 256))
+        return hk_launch_gemm_few_rows(dtype, epi, &a, ctx->stream) ? hk_fail(ctx, HK_ERR_DEVICE, "gemm launch failed") : HK_OK;
     return hk_launch_gemm(dtype, epi, &a, ctx->stream) ? hk_fail(ctx, HK_ERR_DEVICE, "gemm launch failed") : HK_OK;
 }
 

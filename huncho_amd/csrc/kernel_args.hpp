@@ -293,7 +293,7 @@ struct ReadoutArgs {
     int x_f32;                  // x is fp32 (a residual stream kept in fp32) instead of the dtype
 };
 
-// Dense projection Y = X W^T with a fused epilogue (gemm.hip; gemm_split.hip for few rows, which
+// Dense projection Y = X W^T with a fused epilogue (gemm.hip; gemm_few_rows.hip for few rows, which
 // also has EPI_RESIDUAL_F32: fp32 rows of c and y, the fp32 residual stream).
 enum { EPI_STORE = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2, EPI_RESIDUAL_F32 = 3 };
 struct GemmArgs {
@@ -303,7 +303,7 @@ struct GemmArgs {
     void* y;        // [M][N] (EPI_SWIGLU: [M][N / 2])
     long ldx, ldw, ldc, ldy;
     int M, N, K;
-    // gemm_split.hip, EPI_STORE: a second projection of the same x rows, Y2 = X W2^T (row stride of
+    // gemm_few_rows.hip, EPI_STORE: a second projection of the same x rows, Y2 = X W2^T (row stride of
     // w2 = ldw); N2 = 0: none
     const void* w2;
     void* y2;
@@ -338,8 +338,8 @@ int hk_launch_readout(int dtype, const hk::ReadoutArgs* a, hipStream_t st);
 int hk_launch_gdn16_split(int dtype16, const hk::GdnArgs* a, const hk::GdnFusedArgs* fa, int n_seqs, int n_slots,
                           void* scratch, hipStream_t stream);
 int hk_launch_gemm(int dtype16, int epi, const hk::GemmArgs* a, hipStream_t stream);
-float hk_gemm_split_cost(int epi, const hk::GemmArgs* a);
-int hk_launch_gemm_split(int dtype16, int epi, const hk::GemmArgs* a, hipStream_t stream);
+float hk_gemm_few_rows_cost(int epi, const hk::GemmArgs* a);
+int hk_launch_gemm_few_rows(int dtype16, int epi, const hk::GemmArgs* a, hipStream_t stream);
 int hk_launch_lora_merge(int dtype, void* w, long rows, int cols, const float* a, const float* b, int rank, float scale,
                          hipStream_t st);
 int hk_launch_bidir_attention(int dtype, const hk::BertAttnArgs* a, int n_seqs, int max_len, hipStream_t stream);

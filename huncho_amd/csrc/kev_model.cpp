@@ -607,7 +607,7 @@ extern "C" int hk_kev_model_identity(hk_kev_model* m, char* buf, size_t len, siz
          {"recurrent_state_dtype", "fp32"},
          {"causal_conv_execution", f32 || !gdn_mfma || c.conv_k != 4 ? "rocm-gdn-prep-v1" : "rocm-fused-gdn-layer-v1"},
          {"mlp_gate_execution", m->mlp_fused ? "rocm-gemm-swiglu-epilogue-v1" : "rocm-swiglu-v1"},
-         {"projection_kernel", f32 ? "hipblaslt-pinned-or-heuristic-v1" : "rocm-gemm-ksplit-few-rows-or-hipblaslt-v1"},
+         {"projection_kernel", f32 ? "hipblaslt-pinned-or-heuristic-v1" : "rocm-gemm-few-rows-or-hipblaslt-v1"},
          {"pointer_head_dtype", "fp32"},
          {"library", hk_version()}},
         buf, len, needed);

@@ -1,7 +1,7 @@
-"""The few-row GEMM (gemm_split.hip) against a float64 product of the same 16-bit values, through
-hk_linear and through the models' projections, at the edges of its tiles: one row, a row more and
-less than each tile's 32, 64 and 96 rows, K of one to many steps (fewer steps than waves leave a wave
-without any), column counts that leave a part of a tile.
+"""The few-row GEMM (gemm_few_rows.hip) against a float64 product of the same 16-bit values, through
+hk_linear, at the edges of its tiles: one row, a row more and less than each tile's 32, 64, 96 and 128
+rows, K of one to many steps (fewer steps than share a barrier, and not a multiple of them), column
+counts that leave a part of a tile; and its bits against those of many rows, which run on gemm.hip.
 
 Gates: 1 unit in the last place of the dtype (2^-7 relative for bf16, 2^-10 for fp16) plus the fp32
 accumulation's absolute error over K products; the SwiGLU epilogue 2 units, from the rounded gate
@@ -60,11 +60,16 @@ def test_linear_few_rows(ctx, dtype, rows, n, k):
     assert bool(((got - torch.nn.functional.silu(gate) * up).abs() <= tol).all())
 
 
-def test_rows_do_not_depend_on_the_batch(ctx):
-    """K is split the same way for every tile, so a row's result is the same bits at any row count."""
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("epi,n,k", [(0, 1024, 1024), (1, 1024, 3584), (2, 7168, 1024), (1, 768, 1152)])
+def test_rows_do_not_depend_on_the_batch(ctx, dtype, epi, n, k):
+    """An output is one chain of sums over K in order on every path, so a row's result is the same bits
+    in a batch of any size."""
     g = torch.Generator(device="cuda").manual_seed(3)
-    x = torch.randn((600, 1024), generator=g, device="cuda").to(torch.bfloat16)
-    w = (torch.randn((1024, 1024), generator=g, device="cuda") * 0.05).to(torch.bfloat16)
-    whole = linear(ctx, x, w)
-    for rows in (1, 40, 100, 200, 400):
-        assert torch.equal(linear(ctx, x[:rows], w), whole[:rows])
+    x = torch.randn((16384, k), generator=g, device="cuda").to(dtype)
+    w = (torch.randn((n, k), generator=g, device="cuda") * 0.05).to(dtype)
+    c = torch.randn((16384, n), generator=g, device="cuda").to(dtype) if epi == 1 else None
+    cols = n // 2 if epi == 2 else n
+    whole = linear(ctx, x, w, epi, c, cols)  # gemm.hip
+    for rows in (1, 40, 100, 169, 300, 600, 1200):
+        assert torch.equal(linear(ctx, x[:rows], w, epi, c[:rows] if epi == 1 else None, cols), whole[:rows]), rows
