@@ -86,11 +86,11 @@ extern "C" int hk_ctx_destroy(hk_ctx* ctx) {
     hipStreamSynchronize(ctx->stream);
     hk_noalloc_scratch_release(ctx);
     hk_blas_release(ctx);
-    if (ctx->gdn_scratch) {
+    if (ctx->split_scratch) {
         hipDeviceSynchronize();  // its users may be on streams that the context has left
-        hipFree(ctx->gdn_scratch);
+        hipFree(ctx->split_scratch);
     }
-    if (ctx->gdn_moved) hipEventDestroy(ctx->gdn_moved);
+    if (ctx->split_moved) hipEventDestroy(ctx->split_moved);
     if (ctx->fault_dev) hipFree(ctx->fault_dev);
     if (ctx->own_stream) hipStreamDestroy(ctx->own_stream);
     delete ctx;
@@ -100,15 +100,15 @@ extern "C" int hk_ctx_destroy(hk_ctx* ctx) {
 extern "C" int hk_ctx_set_stream(hk_ctx* ctx, void* hip_stream) {
     if (!ctx) return HK_ERR_INVALID;
     const hipStream_t next = (hipStream_t)hip_stream;  // NULL is HIP's null stream
-    if (next != ctx->stream && ctx->gdn_scratch_used) {
+    if (next != ctx->stream && ctx->split_scratch_used) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         const bool ok = hipStreamIsCapturing(ctx->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone &&
-                        (ctx->gdn_moved || hipEventCreateWithFlags(&ctx->gdn_moved, hipEventDisableTiming) == hipSuccess) &&
-                        hipEventRecord(ctx->gdn_moved, ctx->stream) == hipSuccess;
+                        (ctx->split_moved || hipEventCreateWithFlags(&ctx->split_moved, hipEventDisableTiming) == hipSuccess) &&
+                        hipEventRecord(ctx->split_moved, ctx->stream) == hipSuccess;
         (void)hipGetLastError();
-        ctx->gdn_wait = true;
-        ctx->gdn_wait_all = !ok;
-        ctx->gdn_scratch_used = false;
+        ctx->split_wait = true;
+        ctx->split_wait_all = !ok;
+        ctx->split_scratch_used = false;
     }
     ctx->stream = next;
     return HK_OK;
@@ -118,44 +118,44 @@ size_t hk_gdn_split_bytes(int n_tokens, int n_seqs, int heads) {
     return (size_t)(n_tokens / 64 + n_seqs) * heads * hk::HK_GDN_SPLIT_SLOT;
 }
 
-bool hk_gdn_scratch_reserve(hk_ctx* ctx, size_t bytes) {
-    if (bytes <= ctx->gdn_scratch_bytes) return true;
-    if (bytes > kGdnScratchMax) return false;
+bool hk_split_scratch_reserve(hk_ctx* ctx, size_t bytes) {
+    if (bytes <= ctx->split_scratch_bytes) return true;
+    if (bytes > kSplitScratchMax) return false;
     size_t size = 32u << 20;
     while (size < bytes) size <<= 1;
     bytes = size;
-    if (ctx->gdn_scratch) {
+    if (ctx->split_scratch) {
         hipDeviceSynchronize();
-        hipFree(ctx->gdn_scratch);
-        ctx->gdn_scratch = nullptr;
-        ctx->gdn_scratch_bytes = 0;
-        ctx->gdn_scratch_used = ctx->gdn_wait = ctx->gdn_wait_all = false;
+        hipFree(ctx->split_scratch);
+        ctx->split_scratch = nullptr;
+        ctx->split_scratch_bytes = 0;
+        ctx->split_scratch_used = ctx->split_wait = ctx->split_wait_all = false;
     }
-    if (hipMalloc(&ctx->gdn_scratch, bytes) != hipSuccess) {
+    if (hipMalloc(&ctx->split_scratch, bytes) != hipSuccess) {
         (void)hipGetLastError();
-        ctx->gdn_scratch = nullptr;
+        ctx->split_scratch = nullptr;
         return false;
     }
-    ctx->gdn_scratch_bytes = bytes;
+    ctx->split_scratch_bytes = bytes;
     return true;
 }
 
 // The scratch for a call on the context's stream, after the users on other streams, or null: too small
 // (grown only if may_alloc) or the stream is being captured (a graph may be replayed on any stream).
-static void* gdn_scratch_for(hk_ctx* ctx, size_t bytes, bool may_alloc) {
-    if (bytes > (may_alloc ? kGdnScratchMax : ctx->gdn_scratch_bytes)) return nullptr;
+static void* split_scratch_for(hk_ctx* ctx, size_t bytes, bool may_alloc) {
+    if (bytes > (may_alloc ? kSplitScratchMax : ctx->split_scratch_bytes)) return nullptr;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
         (void)hipGetLastError();
         return nullptr;
     }
-    if (!hk_gdn_scratch_reserve(ctx, bytes)) return nullptr;
-    if (ctx->gdn_wait) {
-        if (ctx->gdn_wait_all || hipStreamWaitEvent(ctx->stream, ctx->gdn_moved, 0) != hipSuccess) hipDeviceSynchronize();
-        ctx->gdn_wait = ctx->gdn_wait_all = false;
+    if (!hk_split_scratch_reserve(ctx, bytes)) return nullptr;
+    if (ctx->split_wait) {
+        if (ctx->split_wait_all || hipStreamWaitEvent(ctx->stream, ctx->split_moved, 0) != hipSuccess) hipDeviceSynchronize();
+        ctx->split_wait = ctx->split_wait_all = false;
     }
-    ctx->gdn_scratch_used = true;
-    return ctx->gdn_scratch;
+    ctx->split_scratch_used = true;
+    return ctx->split_scratch;
 }
 
 extern "C" void* hk_ctx_own_stream(hk_ctx* ctx) { return ctx ? (void*)ctx->own_stream : nullptr; }
@@ -477,12 +477,32 @@ extern "C" int hk_paged_kv_write(hk_ctx* ctx, int dtype, const void* k, const vo
                                          head_dim, nullptr, 0, 0, k_pool, v_pool, nullptr);
 }
 
-extern "C" int hk_paged_prefill_attention(hk_ctx* ctx, int dtype, const void* q, long q_tok, long q_head,
-                                          const void* k_pool, const void* v_pool, int num_pages, int page_size,
-                                          const int32_t* bt, int bt_stride, const int32_t* cu, const int32_t* ctxl,
-                                          int n_seqs, int n_tokens, int max_q_len, int q_heads, int kv_heads,
-                                          int head_dim, float scale, const void* gate, long gate_tok, long gate_head,
-                                          void* o, long o_tok, long o_head) {
+// Ranges of a q-block's key tiles for a batch that leaves most of the chip idle (1: not split): ranges of
+// 4 tiles or more, at most kAttnParts workgroups and the 32 ranges that attn_combine takes. Split where
+// the estimates (us, 128-wide heads) favour it by 5 %: a pair of q-blocks runs its tiles at 1.2 us one
+// after another; a range pays 1.25 us a tile (1.75 with two workgroups per CU), and its parts are
+// written and read back. Measured, 16 / 8 heads, unsplit against split:
+//   rows x new tokens over context: 1 x 30 / 1024 24.3 13.3, / 2700 54.8 13.5; 5 x 30 / 2700 55.7 23.1;
+//   16 x 30 / 1024 26.3 25.1, / 4096 81.0 59.9; 4 x 128 / 2048 86.1 30.9; fresh rows 1 x 744 26.4 19.5,
+//   1 x 1024 31.4 25.9, 2 x 1024 32.7 36.6 (not split)
+static const int kAttnParts = 512;
+static int attn_splits(long blocks, long pairs, int tiles, int pair_tiles, bool paired) {
+    if (pairs >= 256 || blocks > kAttnParts / 2) return 1;
+    const int by_tiles = (tiles + 3) / 4, room = (int)(kAttnParts / blocks);
+    const int n = std::min(std::min(by_tiles, room), 32);
+    const int per = (tiles + n - 1) / n;
+    const float whole = 5.0f + 1.18f * pair_tiles + (paired ? 7.0f : 0.0f);
+    const float split = 11.0f + per * (blocks * n > 256 ? 1.75f : 1.25f) + 0.0145f * (float)(blocks * n);
+    return n > 1 && split < 0.95f * whole ? n : 1;
+}
+size_t hk_attn_split_bytes(int head_dim) { return (size_t)kAttnParts * 128 * (head_dim + 2) * sizeof(float); }
+
+int hk_paged_prefill_attention_impl(hk_ctx* ctx, int dtype, const void* q, long q_tok, long q_head, const void* k_pool,
+                                    const void* v_pool, int num_pages, int page_size, const int32_t* bt, int bt_stride,
+                                    const int32_t* cu, const int32_t* ctxl, int n_seqs, int n_tokens, int max_q_len,
+                                    int q_heads, int kv_heads, int head_dim, float scale, const void* gate,
+                                    long gate_tok, long gate_head, void* o, long o_tok, long o_head, int max_ctx,
+                                    bool may_alloc) {
     if (!ctx) return HK_ERR_INVALID;
     if (int rc = check_dtype(ctx, dtype)) return rc;
     if (head_dim < 1 || head_dim > 256)
@@ -531,8 +551,39 @@ extern "C" int hk_paged_prefill_attention(hk_ctx* ctx, int dtype, const void* q,
     hk::AttnArgs a{q, q_tok, q_head, k_pool, v_pool, shift, bt, bt_stride, cu, ctxl, q_heads, kv_heads, group,
                    pos_per_block, scale * 1.4426950408889634f, gate, gate_tok, gate_head, o, o_tok, o_head,
                    num_pages, n_tokens, ctx->fault_dev};
+    if (dtype != HK_F32) {
+        const long most = (long)bt_stride << shift, keys = max_ctx > 0 && max_ctx < most ? max_ctx : most;
+        const int tiles = (int)((keys + 63) / 64 < (1 << 20) ? (keys + 63) / 64 : 1 << 20);
+        const long rows = (long)kv_heads * n_seqs;
+        // a pair's two blocks lie (n_qblocks - 1) x pos_per_block keys apart in all
+        const int pair_tiles = n_qblocks == 1 ? tiles : 2 * tiles - (n_qblocks - 1) * pos_per_block / 64;
+        const int n = attn_splits(rows * n_qblocks, rows * ((n_qblocks + 1) / 2), tiles, pair_tiles, n_qblocks > 1);
+        const size_t bytes = (size_t)(rows * n_qblocks * n) * 128 * (head_dim + 2) * sizeof(float);
+        if (n > 1) {
+            if (void* scratch = split_scratch_for(ctx, bytes, may_alloc)) {
+                a.n_split = n;
+                a.split_tiles = 4;
+                a.n_qblocks = n_qblocks;
+                a.part = (float*)scratch;
+                a.part_ml = a.part + (size_t)(rows * n_qblocks * n) * 128 * head_dim;
+                const int rc = hk_launch_paged_prefill_attention_split(dtype, &a, head_dim, n_seqs, ctx->stream);
+                return rc ? hk_fail(ctx, rc, "attention launch failed") : HK_OK;
+            }
+        }
+    }
     int rc = hk_launch_paged_prefill_attention(dtype, &a, head_dim, n_seqs, n_qblocks, ctx->stream);
     return rc ? hk_fail(ctx, rc, "attention launch failed") : HK_OK;
+}
+
+extern "C" int hk_paged_prefill_attention(hk_ctx* ctx, int dtype, const void* q, long q_tok, long q_head,
+                                          const void* k_pool, const void* v_pool, int num_pages, int page_size,
+                                          const int32_t* bt, int bt_stride, const int32_t* cu, const int32_t* ctxl,
+                                          int n_seqs, int n_tokens, int max_q_len, int q_heads, int kv_heads,
+                                          int head_dim, float scale, const void* gate, long gate_tok, long gate_head,
+                                          void* o, long o_tok, long o_head) {
+    return hk_paged_prefill_attention_impl(ctx, dtype, q, q_tok, q_head, k_pool, v_pool, num_pages, page_size, bt,
+                                           bt_stride, cu, ctxl, n_seqs, n_tokens, max_q_len, q_heads, kv_heads, head_dim,
+                                           scale, gate, gate_tok, gate_head, o, o_tok, o_head, 0, true);
 }
 
 int hk_gated_delta_chunked_rows(hk_ctx* ctx, int dtype, const void* q, long q_tok, const void* k, long k_tok,
@@ -688,7 +739,7 @@ int hk_gdn_fused_rows(hk_ctx* ctx, int dtype, const void* mixed, long mixed_tok,
     hk::GdnFusedArgs fa{mixed, mixed_tok, conv_w, (int)conv_dim, conv_hist, conv_tail_out, ba, ba_tok, b_col, a_col,
                         base_g, dt_bias, 1.0f / sqrtf(128.0f), k_heads, z, z_tok, norm_w, eps, hist_rows, tail_rows};
     if (gdn_split_takes(n_seqs, n_tokens, heads)) {
-        if (void* scratch = gdn_scratch_for(ctx, hk_gdn_split_bytes(n_tokens, n_seqs, heads), may_alloc)) {
+        if (void* scratch = split_scratch_for(ctx, hk_gdn_split_bytes(n_tokens, n_seqs, heads), may_alloc)) {
             const int rc = hk_launch_gdn16_split(dtype, &a, &fa, n_seqs, n_tokens / 64 + n_seqs, scratch, ctx->stream);
             return rc ? hk_fail(ctx, rc, "fused Gated DeltaNet launch failed") : HK_OK;
         }

@@ -85,6 +85,15 @@ __device__ __forceinline__ int swz(int r) { return 4 * (r & 3); }
 __device__ __forceinline__ int swzk(int r) { return (r & 7) | (((r >> 4) & 1) << 3); }
 __device__ __forceinline__ int lds_off_k(int r, int c) { return r * KV_ROW + 8 * (c ^ swzk(r)); }
 
+// Key-split launches: tiles per range of a q-block of nt tiles (nt: one range), and the first part of a
+// q-block. The same in the attention and the combining kernel.
+__device__ __forceinline__ int split_range(const AttnArgs& a, int nt) {
+    return min(nt, max(a.split_tiles, (nt + a.n_split - 1) / a.n_split));
+}
+__device__ __forceinline__ long part_index(const AttnArgs& a, int seq, int qb, int kvh) {
+    return (((long)seq * a.n_qblocks + qb) * a.kv_heads + kvh) * a.n_split;
+}
+
 // Pipeline per 64-key tile (one barrier per tile): issue the direct-to-LDS copies of tile
 // t+1 into buffer (t+1) % 2 (page read one tile earlier) and the block-table read of tile
 // t+2; S^T = K Q^T, online softmax and O^T += V^T P^T on buffer t % 2; wait for this wave's
@@ -94,7 +103,13 @@ __device__ __forceinline__ int lds_off_k(int r, int c) { return r * KV_ROW + 8 *
 // (otherwise p <= 2^8 and the fp32 sums lose nothing), which is the same normalised result.
 // The row sum l adds the probabilities as rounded for P.V (v_dot2 against ones), so the
 // weights applied to V sum to one.
-template <typename T, int NH>
+//
+// SPLIT: a batch of few rows leaves most CUs idle (five 30-token questions over one 2,700-token state:
+// 40 workgroups of 43 tiles, 55.7 us; split 17.4 + 6.1). Then a workgroup takes one q-block and one range of its key tiles,
+// and writes its unnormalised fp32 O rows with their max and sum; attn_combine adds the ranges of a
+// row in their order. A q-block with a single range is finished here as in the unsplit kernel. A range
+// may lie past a row's last visible key: its max stays -inf and its probabilities 0.
+template <typename T, int NH, bool SPLIT>
 __global__ __launch_bounds__(256, NH == 1 ? 2 : 1) void paged_prefill_attn_16(AttnArgs a) {
     typedef typename Mma16<T>::v8 v8;
     typedef typename Mma16<T>::v4 v4;
@@ -110,7 +125,7 @@ __global__ __launch_bounds__(256, NH == 1 ? 2 : 1) void paged_prefill_attn_16(At
     // and consecutive ids go round-robin to the 8 XCDs, so all q-block pairs of one
     // (sequence, KV head) run together on one XCD and share its L2 copy of the K/V pages
     const int kvh = blockIdx.x;
-    const int z = blockIdx.y;
+    const int z = SPLIT ? 0 : blockIdx.y;
     const int seq = blockIdx.z;
     const int q0 = a.cu_seqlens_q[seq];
     const int q_len = a.cu_seqlens_q[seq + 1] - q0;
@@ -124,14 +139,19 @@ __global__ __launch_bounds__(256, NH == 1 ? 2 : 1) void paged_prefill_attn_16(At
     // this workgroup's q-blocks: the mirrored pair (nq - 1 - z, z), so every workgroup of a
     // sequence runs nq + 1 key tiles; the longer block goes first
     const int nq = (q_len + P - 1) / P;
-    if (2 * z >= nq) return;
-    const int qb_a = nq - 1 - z, qb_b = z;
-    const int n_blocks = qb_a == qb_b ? 1 : 2;
+    // (SPLIT: q-blocks past n_qblocks, rows longer than max_q_len, have no part)
+    const int qb_a = SPLIT ? a.n_qblocks - 1 - (int)(blockIdx.y / a.n_split) : nq - 1 - z, qb_b = z;
+    if (SPLIT ? qb_a >= nq : 2 * z >= nq) return;
+    const int n_blocks = SPLIT || qb_a == qb_b ? 1 : 2;
     const int off = ctx - q_len;  // absolute position of the first new query
     const int* table = a.block_tables + (long)seq * a.bt_stride;
     const int pmask = (1 << a.page_shift) - 1;
     auto block_tiles = [&](int qb) { return (off + min(q_len, (qb + 1) * P) - 1) / BN + 1; };
-    const int nt_a = block_tiles(qb_a);
+    // SPLIT: tiles i0 .. nt_a - 1 of the block's
+    const int nt_all = block_tiles(qb_a), range = SPLIT ? split_range(a, nt_all) : nt_all;
+    const int i0 = SPLIT ? (int)(blockIdx.y % a.n_split) * range : 0;
+    if (SPLIT && i0 >= nt_all) return;
+    const int nt_a = SPLIT ? min(nt_all, i0 + range) : nt_all;
     const int n_sched = nt_a + (n_blocks == 2 ? block_tiles(qb_b) : 0);
     // schedule step i -> key tile: block a's tiles 0..nt_a-1, then block b's from 0
     auto sched_tile = [&](int i) { return i < nt_a ? i : i - nt_a; };
@@ -321,7 +341,7 @@ __global__ __launch_bounds__(256, NH == 1 ? 2 : 1) void paged_prefill_attn_16(At
     };
     // probabilities of one half as the P.V operand (rounded to T), and their row sums
     auto half_p = [&](const f32x16& sv, v8* pf) {
-        const float mc = m_use * c;
+        const float mc = SPLIT && m_use == -INFINITY ? 0.0f : m_use * c;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             v8 t;
@@ -403,11 +423,11 @@ __global__ __launch_bounds__(256, NH == 1 ? 2 : 1) void paged_prefill_attn_16(At
     std::integral_constant<bool, true> with_mask;
 
     begin_block(qb_a);
-    lookup(0);  // issued before Q, so that resolving it waits for the table read alone
+    lookup(i0);  // issued before Q, so that resolving it waits for the table read alone
     load_q(qb_a);
     resolve();
-    load_tile(0, 0);
-    lookup(sched_tile(min(1, n_sched - 1)));
+    load_tile(i0, i0 & 1);
+    lookup(sched_tile(min(i0 + 1, n_sched - 1)));
     __builtin_amdgcn_s_waitcnt(VMCNT0);  // Q and this wave's copies of tile 0
     __syncthreads();
     // The two blocks run as two loops whose bodies issue only the tile and table loads:
@@ -415,8 +435,22 @@ __global__ __launch_bounds__(256, NH == 1 ? 2 : 1) void paged_prefill_attn_16(At
     // holds a tile's S^T behind the next tile's prefetch.
     {
         const int mf = min(mask_from(qb_a), nt_a);
-        for (int i = 0; i < mf; ++i) step(i, no_mask);
-        for (int i = mf; i < nt_a; ++i) step(i, with_mask);
+        for (int i = i0; i < mf; ++i) step(i, no_mask);
+        for (int i = max(mf, i0); i < nt_a; ++i) step(i, with_mask);
+    }
+    if (SPLIT && range < nt_all) {
+        const float l_tot = l_run + __shfl_xor(l_run, 32);
+        if (!q_valid) return;  // rows past the sequence have no part (short suffixes fill half a block)
+        const long w = part_index(a, seq, qb_a, kvh) + blockIdx.y % a.n_split;
+        float* const op = a.part + (w * 128 + row) * HD + 4 * g;
+#pragma unroll
+        for (int db = 0; db < 4 * NH; ++db)
+#pragma unroll
+            for (int jj = 0; jj < 4; ++jj)
+                *(f32x4*)(op + 32 * db + 8 * jj) = f32x4{acc_o[db][4 * jj], acc_o[db][4 * jj + 1], acc_o[db][4 * jj + 2],
+                                                         acc_o[db][4 * jj + 3]};
+        if (g == 0) *(f32x2*)(a.part_ml + (w * 128 + row) * 2) = f32x2{m_use, l_tot};
+        return;
     }
     if (n_blocks == 2) load_q(qb_b);  // lands while block a's output is written
     finish_block(qb_a, (nt_a - 1) & 1);  // the buffer of block a's last tile is free
@@ -428,6 +462,57 @@ __global__ __launch_bounds__(256, NH == 1 ? 2 : 1) void paged_prefill_attn_16(At
         for (int i = mf; i < n_sched; ++i) step(i, with_mask);
         finish_block(qb_b, 0);
     }
+}
+
+// Adds the key ranges of RPP query rows of a q-block in their order and finishes them as the attention
+// kernel does: o = sum_s 2^((m_s - m) c) O_s / l, rounded to T, times the gate. HD / 4 lanes per row.
+template <typename T, int NH>
+__global__ __launch_bounds__(256) void attn_combine(AttnArgs a) {
+    typedef typename Mma16<T>::v4 v4;
+    constexpr int HD = 128 * NH, LPR = HD / 4, RPP = 256 / LPR;  // lanes per row, rows per pass
+    const int kvh = blockIdx.x, qb = blockIdx.y / (128 / RPP), seq = blockIdx.z;
+    const int q0 = a.cu_seqlens_q[seq], q_len = a.cu_seqlens_q[seq + 1] - q0, ctx = a.context_lens[seq];
+    const int P = a.pos_per_block;
+    if (q0 < 0 || q_len < 0 || q0 + q_len > a.n_tokens || q_len > ctx || qb * P >= q_len) return;
+    const int nt = (ctx - q_len + min(q_len, (qb + 1) * P) - 1) / BN + 1, range = split_range(a, nt);
+    if (range >= nt) return;  // finished by the attention kernel
+    const int ns = (nt + range - 1) / range;
+    const long w0 = part_index(a, seq, qb, kvh);
+    const int row = RPP * (blockIdx.y % (128 / RPP)) + threadIdx.x / LPR, d = 4 * (threadIdx.x % LPR);
+    const int qi = qb * P + (row & (P - 1)), head = kvh * a.group + row / P;
+    if (qi >= q_len) return;  // the same for a row's lanes
+    // lane i of each 32 holds range i's max and sum: one load, then the weights by shuffle
+    const int i = threadIdx.x & 31;
+    const f32x2 v = *((const f32x2*)a.part_ml + (w0 + min(i, ns - 1)) * 128 + row);
+    float m = i < ns ? v[0] : -INFINITY;
+#pragma unroll
+    for (int x = 1; x < 32; x <<= 1) m = fmaxf(m, __shfl_xor(m, x));
+    // a range without a visible key adds nothing (also -inf - -inf); a NaN or +inf max stays one
+    const float wgt = i >= ns || v[0] == -INFINITY ? 0.0f : fast_exp2((v[0] - m) * a.scale_log2);
+    float l = i < ns ? wgt * v[1] : 0.0f;
+#pragma unroll
+    for (int x = 1; x < 32; x <<= 1) l += __shfl_xor(l, x);
+    const float* const op = a.part + (w0 * 128 + row) * HD + d;
+    f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < ns; s0 += 8) {  // 8 loads in flight
+        f32x4 t[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) t[e] = *(const f32x4*)(op + (long)min(s0 + e, ns - 1) * 128 * HD);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float w = __shfl(wgt, s0 + e, 32);
+            if (s0 + e < ns) o += w * t[e];
+        }
+    }
+    const float inv = 1.0f / l;
+    const long tok = q0 + qi;
+    v4 r = v4{(T)(o[0] * inv), (T)(o[1] * inv), (T)(o[2] * inv), (T)(o[3] * inv)};
+    if (a.gate) {
+        const v4 gv = *(const v4*)((const T*)a.gate + tok * a.g_tok + (long)head * a.g_head + d);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r[e] = (T)((float)r[e] * (float)(T)fast_sigmoid((float)gv[e]));
+    }
+    *(v4*)((T*)a.o + tok * a.o_tok + (long)head * a.o_head + d) = r;
 }
 
 // ---------------------------------------------------------------------------
@@ -599,13 +684,13 @@ extern "C" int hk_launch_paged_prefill_attention(int dtype, const hk::AttnArgs* 
     // set once, under C++'s thread-safe static initialisation (replicas launch from several threads);
     // head width 256 holds two 128-wide halves per K / V tile: 131,072 B, one workgroup per CU
     static const bool configured =
-        hipFuncSetAttribute((const void*)paged_prefill_attn_16<bf16, 1>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        hipFuncSetAttribute((const void*)paged_prefill_attn_16<bf16, 1, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)ATTN16_LDS) == hipSuccess &&
-        hipFuncSetAttribute((const void*)paged_prefill_attn_16<f16, 1>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        hipFuncSetAttribute((const void*)paged_prefill_attn_16<f16, 1, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)ATTN16_LDS) == hipSuccess &&
-        hipFuncSetAttribute((const void*)paged_prefill_attn_16<bf16, 2>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        hipFuncSetAttribute((const void*)paged_prefill_attn_16<bf16, 2, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)(2 * ATTN16_LDS)) == hipSuccess &&
-        hipFuncSetAttribute((const void*)paged_prefill_attn_16<f16, 2>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        hipFuncSetAttribute((const void*)paged_prefill_attn_16<f16, 2, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)(2 * ATTN16_LDS)) == hipSuccess;
     if (!configured) return HK_ERR_DEVICE;
     // 16-bit: one workgroup per mirrored pair of q-blocks (head width 128 or 256); fp32: one per
@@ -621,14 +706,37 @@ extern "C" int hk_launch_paged_prefill_attention(int dtype, const hk::AttnArgs* 
     const bool bf = dtype == DT_BF16;
     if (head_dim == 128) {
         if (bf)
-            hipLaunchKernelGGL((paged_prefill_attn_16<bf16, 1>), grid, dim3(256), ATTN16_LDS, stream, *args);
+            hipLaunchKernelGGL((paged_prefill_attn_16<bf16, 1, false>), grid, dim3(256), ATTN16_LDS, stream, *args);
         else
-            hipLaunchKernelGGL((paged_prefill_attn_16<f16, 1>), grid, dim3(256), ATTN16_LDS, stream, *args);
+            hipLaunchKernelGGL((paged_prefill_attn_16<f16, 1, false>), grid, dim3(256), ATTN16_LDS, stream, *args);
     } else {
         if (bf)
-            hipLaunchKernelGGL((paged_prefill_attn_16<bf16, 2>), grid, dim3(256), 2 * ATTN16_LDS, stream, *args);
+            hipLaunchKernelGGL((paged_prefill_attn_16<bf16, 2, false>), grid, dim3(256), 2 * ATTN16_LDS, stream, *args);
         else
-            hipLaunchKernelGGL((paged_prefill_attn_16<f16, 2>), grid, dim3(256), 2 * ATTN16_LDS, stream, *args);
+            hipLaunchKernelGGL((paged_prefill_attn_16<f16, 2, false>), grid, dim3(256), 2 * ATTN16_LDS, stream, *args);
     }
     return hipGetLastError() == hipSuccess ? HK_OK : HK_ERR_DEVICE;
+}
+
+template <typename T, int NH>
+static int launch_split(const hk::AttnArgs* a, int n_seqs, hipStream_t stream) {
+    using namespace hk;
+    auto kern = paged_prefill_attn_16<T, NH, true>;
+    static const bool configured = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                       (int)(NH * ATTN16_LDS)) == hipSuccess;
+    if (!configured) return HK_ERR_DEVICE;
+    hipLaunchKernelGGL(kern, dim3(a->kv_heads, a->n_qblocks * a->n_split, n_seqs), dim3(256), NH * ATTN16_LDS, stream, *a);
+    hipLaunchKernelGGL((attn_combine<T, NH>), dim3(a->kv_heads, a->n_qblocks * (128 / (NH == 1 ? 8 : 4)), n_seqs), dim3(256), 0,
+                       stream, *a);
+    return hipGetLastError() == hipSuccess ? HK_OK : HK_ERR_DEVICE;
+}
+
+// 16-bit types, head_dim 128 or 256; the caller has sized part and part_ml
+extern "C" int hk_launch_paged_prefill_attention_split(int dtype, const hk::AttnArgs* a, int head_dim, int n_seqs,
+                                                       hipStream_t stream) {
+    if (head_dim == 128)
+        return dtype == hk::DT_BF16 ? launch_split<hk::bf16, 1>(a, n_seqs, stream) : launch_split<hk::f16, 1>(a, n_seqs, stream);
+    if (head_dim == 256)
+        return dtype == hk::DT_BF16 ? launch_split<hk::bf16, 2>(a, n_seqs, stream) : launch_split<hk::f16, 2>(a, n_seqs, stream);
+    return HK_ERR_UNSUPPORTED;
 }

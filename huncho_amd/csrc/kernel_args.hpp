@@ -25,6 +25,11 @@ struct AttnArgs {
     int num_pages;
     int n_tokens;
     int* fault;
+    // key-split kernel: each q-block's tiles in at most n_split ranges of at least split_tiles; part holds
+    // the ranges' unnormalised fp32 O rows, part_ml their (row max, row sum) pairs
+    int n_split, split_tiles, n_qblocks;
+    float* part;
+    float* part_ml;
 };
 
 struct GdnArgs {
@@ -316,6 +321,8 @@ struct GemmArgs {
 extern "C" {
 int hk_launch_paged_prefill_attention(int dtype, const hk::AttnArgs* args, int head_dim, int n_seqs, int n_qblocks,
                                       hipStream_t stream);
+int hk_launch_paged_prefill_attention_split(int dtype, const hk::AttnArgs* args, int head_dim, int n_seqs,
+                                            hipStream_t stream);
 int hk_launch_gated_delta_chunked(int dtype, const hk::GdnArgs* args, int n_seqs, hipStream_t stream);
 int hk_launch_gdn16(int dtype16, int fused, const hk::GdnArgs* a, const hk::GdnFusedArgs* fa, int n_seqs,
                     hipStream_t stream);

@@ -30,6 +30,8 @@
 //     complete, and is retained when it completes.
 #include <string.h>
 
+#include <algorithm>
+
 #include <deque>
 #include <map>
 #include <unordered_map>
@@ -411,6 +413,7 @@ static int forward_cached(hk_kev_cache* c, const uint64_t* handles_host, int n_s
         return rollback(hk_fail(ctx, HK_ERR_DEVICE, "cache table upload failed"));
     KevCacheView view;
     view.ctx_lens_dev = lens_dev;
+    view.max_ctx = *std::max_element(lens.begin(), lens.end());
     view.k_pools = c->k_pools;
     view.v_pools = c->v_pools;
     for (int g = 0; g < c->n_gdn; ++g) {

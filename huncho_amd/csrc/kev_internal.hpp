@@ -47,6 +47,7 @@ struct hk_kev_model {
 // Per-call view of cached state for a continuation forward (all pointers owned by the cache).
 struct KevCacheView {
     const int32_t* ctx_lens_dev;         // [n_seqs] cached + new tokens per sequence
+    int max_ctx = 0;                     // the longest of them
     std::vector<void*> k_pools, v_pools;  // one pool per attention layer, in layer order
     // one device array of n_seqs pointers per Gated DeltaNet layer, in layer order
     std::vector<const float* const*> init_rows;

@@ -229,11 +229,13 @@ extern "C" int hk_kev_model_create(hk_ctx* ctx, int dtype, const hk_kev_config* 
         hk_rope_fill_table(c.rotary_dim, c.rope_theta, c.max_context, dtype, cs.data(), sn.data());
         if ((rc = upload_f32(m, cs, &m->rope_cos)) || (rc = upload_f32(m, sn, &m->rope_sin))) return fail(rc);
     }
-    // scratch for up to four rows of max_context tokens through the Gated DeltaNet layers, at most half
-    // of the limit, so that no forward allocates (batches that do not fit run the layer without it)
+    // scratch for the key-split attention, and for up to four rows of max_context tokens through the Gated
+    // DeltaNet layers, at most half of the limit, so that no forward allocates (batches that do not fit
+    // run the layer without it)
+    if (dtype != HK_F32 && (c.head_dim == 128 || c.head_dim == 256)) hk_split_scratch_reserve(ctx, hk_attn_split_bytes(c.head_dim));
     if (dtype != HK_F32 && c.conv_k == 4 && c.lin_key_dim == 128 && c.lin_v_dim == 128) {
         const size_t want = hk_gdn_split_bytes(4 * (c.max_context < 65536 ? c.max_context : 65536), 4, c.lin_n_v_heads);
-        hk_gdn_scratch_reserve(ctx, want < kGdnScratchMax / 2 ? want : kGdnScratchMax / 2);
+        hk_split_scratch_reserve(ctx, want < kSplitScratchMax / 2 ? want : kSplitScratchMax / 2);
     }
     hipStreamSynchronize(nullptr);  // the weight copies, on the null stream, are complete before the
                                     // context's stream (non-blocking) uses them
@@ -509,10 +511,10 @@ int kev_forward_impl(hk_kev_model* m, const int32_t* ids, const int32_t* cu_dev,
                                               c.eps, m->rope_cos, m->rope_sin, c.rotary_dim, c.max_context, cu_dev,
                                               ctx_lens, n_seqs, n, bt, bt_stride, num_pages, c.page_size, Hq, Hkv, hd,
                                               qg, rows, 2 * hd, k_pool, v_pool, b.tok_sp));
-            RUN(hk_paged_prefill_attention(ctx, dt, qg, rows, 2 * hd, k_pool, v_pool, num_pages, c.page_size, bt,
-                                           bt_stride, cu_dev, ctx_lens, n_seqs, n, max_len, Hq, Hkv, hd,
-                                           (float)(1.0 / sqrt((double)hd)), qg + (size_t)hd * e, rows, 2 * hd, b.o,
-                                           (long)Hq * hd, hd));
+            RUN(hk_paged_prefill_attention_impl(ctx, dt, qg, rows, 2 * hd, k_pool, v_pool, num_pages, c.page_size, bt,
+                                                bt_stride, cu_dev, ctx_lens, n_seqs, n, max_len, Hq, Hkv, hd,
+                                                (float)(1.0 / sqrt((double)hd)), qg + (size_t)hd * e, rows, 2 * hd, b.o,
+                                                (long)Hq * hd, hd, view ? view->max_ctx : max_len, false));
             RUN(hk_gemm_xwt_cd(ctx, dt, xdt, n, H, Hq * hd, b.o, Hq * hd, L.w_o, Hq * hd, b.x, H, b.x, H, 1.0f, 1.0f));
         }
         RUN(norm_x(m, b.x, L.post_norm, n, b.h));

@@ -1,0 +1,105 @@
+"""The key-split paged attention (few rows over long contexts) against float64 attention over the same
+16-bit values: contexts that end on, before and after a 64-key tile, one and several q-blocks, rows too
+short to be split beside long ones, both head widths, groups of 1 to 8, shared pages, with and without
+the gate.
+
+Tolerance (2-norm): a probability, the output, the gate and their product are each rounded once to the
+dtype, an rms of 2^-9 / sqrt(3) (bf16) or 2^-12 / sqrt(3) (fp16) per rounding: 2.3e-3 and 2.8e-4 for
+four; twice that."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from huncho_amd.ops import paged_prefill_attention
+
+pytestmark = pytest.mark.gpu
+
+TOL = {torch.bfloat16: 4.6e-3, torch.float16: 5.6e-4}
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from huncho_amd.ops import context_for_torch
+
+    c = context_for_torch(0)
+    yield c
+    c.close()
+
+
+def run(ctx, q_lens, ctx_lens, hq, hkv, d, page, dtype, gate, seed, spare=0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    r = lambda *s: torch.randn(s, generator=g, device="cuda").to(dtype)
+    n, rows = sum(q_lens), len(q_lens)
+    need = [(c + page - 1) // page for c in ctx_lens]
+    perm = np.random.default_rng(seed).permutation(sum(need)).astype(np.int32)
+    bt = np.zeros((rows, max(need) + spare), np.int32)
+    at = 0
+    for s, m in enumerate(need):
+        bt[s, :m] = perm[at:at + m]
+        at += m
+    kp, vp = r(sum(need), hkv, page, d), r(sum(need), hkv, page, d)
+    qg = r(n, hq, 2 * d)
+    q, gt = qg[:, :, :d], qg[:, :, d:]
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(q_lens)]), dtype=torch.int32, device="cuda")
+    lens = torch.tensor(ctx_lens, dtype=torch.int32, device="cuda")
+    o = paged_prefill_attention(ctx, q, kp, vp, torch.from_numpy(bt).cuda(), cu, lens, max(q_lens),
+                                gate=gt if gate else None)
+    assert ctx.take_faults() == 0
+    refs, t0 = [], 0
+    for s, (L, c) in enumerate(zip(q_lens, ctx_lens)):
+        pages = torch.from_numpy(bt[s, :need[s]].astype(np.int64)).cuda()
+        kk = kp[pages].transpose(1, 2).reshape(-1, hkv, d)[:c].double().repeat_interleave(hq // hkv, 1)
+        vv = vp[pages].transpose(1, 2).reshape(-1, hkv, d)[:c].double().repeat_interleave(hq // hkv, 1)
+        qq = q[t0:t0 + L].double().transpose(0, 1).contiguous()
+        sc = qq @ kk.permute(1, 2, 0).contiguous() / math.sqrt(d)
+        pos = torch.arange(c - L, c, device="cuda")
+        sc.masked_fill_(torch.arange(c, device="cuda")[None] > pos[:, None], -math.inf)
+        ref = (sc.softmax(-1) @ vv.transpose(0, 1).contiguous()).transpose(0, 1)
+        refs.append(ref * torch.sigmoid(gt[t0:t0 + L].double()) if gate else ref)
+        t0 += L
+    ref = torch.cat(refs)
+    return o, float((o.double() - ref).norm() / ref.norm())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("gate", [False, True])
+@pytest.mark.parametrize("q_lens,ctx_lens,hq,hkv,d,page", [
+    ([1], [1024], 16, 8, 128, 16), ([30, 20, 40], [2700, 2701, 2751], 16, 8, 128, 16), ([1], [4097], 8, 8, 128, 64),
+    ([64, 3], [2048, 10], 16, 8, 128, 16), ([65], [1985], 16, 8, 128, 32), ([1500], [1500], 16, 8, 128, 16),
+    ([200, 1, 700], [900, 3000, 700], 16, 2, 128, 16), ([33], [3000], 8, 2, 256, 16), ([700], [1300], 16, 4, 256, 16)])
+def test_split_matches_float64(ctx, dtype, gate, q_lens, ctx_lens, hq, hkv, d, page):
+    _, e = run(ctx, q_lens, ctx_lens, hq, hkv, d, page, dtype, gate, sum(q_lens) + sum(ctx_lens))
+    assert e < TOL[dtype], e
+
+
+def test_short_context_under_a_wide_table(ctx):
+    """The ranges follow the context, not the table's width: a short row is not split, and gives the same
+    bits as under a table of its own size."""
+    a, _ = run(ctx, [20], [150], 16, 8, 128, 16, torch.bfloat16, True, 5)
+    b, e = run(ctx, [20], [150], 16, 8, 128, 16, torch.bfloat16, True, 5, spare=500)
+    assert torch.equal(a, b) and e < TOL[torch.bfloat16]
+
+
+def test_nan_and_infinite_scores(ctx):
+    """A key whose scores are +inf or NaN makes its rows NaN, as softmax does, in whichever range it lies;
+    keys past a row's position do not reach it."""
+    g = torch.Generator(device="cuda").manual_seed(2)
+    c, L = 2000, 8
+    kp = torch.randn((125, 8, 16, 128), generator=g, device="cuda").to(torch.bfloat16)
+    vp = torch.randn((125, 8, 16, 128), generator=g, device="cuda").to(torch.bfloat16)
+    q = torch.rand((L, 16, 128), generator=g, device="cuda").to(torch.bfloat16) + 0.1
+    bt = torch.arange(125, dtype=torch.int32, device="cuda").view(1, -1)
+    cu = torch.tensor([0, L], dtype=torch.int32, device="cuda")
+    lens = torch.tensor([c], dtype=torch.int32, device="cuda")
+    for key, val in ((1000, math.inf), (300, math.nan)):
+        k2 = kp.clone()
+        k2[key // 16, 0, key % 16] = val
+        o = paged_prefill_attention(ctx, q, k2, vp, bt, cu, lens, L)
+        assert bool(o[:, :2].isnan().all()) and not bool(o[:, 2:].isnan().any())
+    k2 = kp.clone()
+    k2[124, :, 15] = math.inf  # key 1999: visible to the last row alone
+    o = paged_prefill_attention(ctx, q, k2, vp, bt, cu, lens, L)
+    assert not bool(o[:-1].isnan().any()) and bool(o[-1].isnan().all())
+    ctx.take_faults()
