@@ -478,13 +478,14 @@ extern "C" int hk_paged_kv_write(hk_ctx* ctx, int dtype, const void* k, const vo
 }
 
 // Ranges of a q-block's key tiles for a batch that leaves most of the chip idle (1: not split): ranges of
-// 4 tiles or more, at most kAttnParts workgroups and the 32 ranges that attn_combine takes. Split where
-// the estimates (us, 128-wide heads) favour it by 5 %: a pair of q-blocks runs its tiles at 1.2 us one
-// after another; a range pays 1.25 us a tile (1.75 with two workgroups per CU), and its parts are
-// written and read back. Measured, 16 / 8 heads, unsplit against split:
-//   rows x new tokens over context: 1 x 30 / 1024 24.3 13.3, / 2700 54.8 13.5; 5 x 30 / 2700 55.7 23.1;
-//   16 x 30 / 1024 26.3 25.1, / 4096 81.0 59.9; 4 x 128 / 2048 86.1 30.9; fresh rows 1 x 744 26.4 19.5,
-//   1 x 1024 31.4 25.9, 2 x 1024 32.7 36.6 (not split)
+// 4 tiles or more, at most kAttnParts workgroups and the 32 ranges that attn_combine takes. Only for
+// suffixes, contexts of 1,024 tokens or more and at least four times as long as the rows: the sums of
+// split rows round differently, and a prefix computed alone keeps the bits that it has in a large batch.
+// There, where the estimates (us, 128-wide heads) favour it by 5 %: a pair of q-blocks runs its tiles at
+// 1.2 us one after another; a range pays 1.25 us a tile (1.75 with two workgroups per CU), and its parts
+// are written and read back. Measured, 16 / 8 heads, unsplit against split, rows x new tokens / context:
+//   1 x 30 / 1024 24.3 12.8, / 2700 54.8 13.5; 5 x 30 / 2700 55.7 23.1; 16 x 30 / 1024 26.3 26.8 (not
+//   split), / 4096 81.0 56.7; 4 x 128 / 2048 86.1 28.5
 static const int kAttnParts = 512;
 static int attn_splits(long blocks, long pairs, int tiles, int pair_tiles, bool paired) {
     if (pairs >= 256 || blocks > kAttnParts / 2) return 1;
@@ -557,7 +558,9 @@ int hk_paged_prefill_attention_impl(hk_ctx* ctx, int dtype, const void* q, long 
         const long rows = (long)kv_heads * n_seqs;
         // a pair's two blocks lie (n_qblocks - 1) x pos_per_block keys apart in all
         const int pair_tiles = n_qblocks == 1 ? tiles : 2 * tiles - (n_qblocks - 1) * pos_per_block / 64;
-        const int n = attn_splits(rows * n_qblocks, rows * ((n_qblocks + 1) / 2), tiles, pair_tiles, n_qblocks > 1);
+        const int n = tiles < 16 || keys / 4 < max_q_len
+                          ? 1
+                          : attn_splits(rows * n_qblocks, rows * ((n_qblocks + 1) / 2), tiles, pair_tiles, n_qblocks > 1);
         const size_t bytes = (size_t)(rows * n_qblocks * n) * 128 * (head_dim + 2) * sizeof(float);
         if (n > 1) {
             if (void* scratch = split_scratch_for(ctx, bytes, may_alloc)) {
@@ -586,11 +589,23 @@ extern "C" int hk_paged_prefill_attention(hk_ctx* ctx, int dtype, const void* q,
                                            scale, gate, gate_tok, gate_head, o, o_tok, o_head, 0, true);
 }
 
+// Whether the fp32 delta rule takes its three-kernel form (delta_rule_split.hip): few chains (pairs of a
+// row and a head) of a chunk or more on average. Measured, 16 heads, us, one kernel against three, by rows
+// x tokens: 1 x 64 37.6 26.6, x 512 256 54.3, x 2048 1055 153;  4 x 64 38.0 32.1, x 512 269 111;  8 x 64
+// 39.9 47.7 (not split), x 128 73.4 64.3, x 1024 571 443
+static bool delta_split_takes(int n_seqs, int n_tokens, int heads) {
+    const long chains = (long)n_seqs * heads, chunks = n_tokens / 64;
+    return chains <= 64 ? chunks >= n_seqs : chains <= 128 && chunks >= 2L * n_seqs;
+}
+size_t hk_delta_split_bytes(int n_tokens, int n_seqs, int heads) {
+    return (size_t)(n_tokens / 64 + n_seqs) * heads * hk::HK_DELTA_SPLIT_SLOT;
+}
+
 int hk_gated_delta_chunked_rows(hk_ctx* ctx, int dtype, const void* q, long q_tok, const void* k, long k_tok,
                                 const void* v, long v_tok, const float* g, const float* beta, const int32_t* cu,
                                 int n_seqs, int n_tokens, int heads, int k_heads, int dk, int dv,
                                 const float* initial_state, float* final_state, void* o, long o_tok,
-                                const float* const* init_rows, float* const* final_rows) {
+                                const float* const* init_rows, float* const* final_rows, bool may_alloc) {
     if (!ctx) return HK_ERR_INVALID;
     if (int rc = check_dtype(ctx, dtype)) return rc;
     // 128 x 128 states on the chunked MFMA kernels, others (each width in 1..256, at most 32768
@@ -613,6 +628,13 @@ int hk_gated_delta_chunked_rows(hk_ctx* ctx, int dtype, const void* q, long q_to
     hipSetDevice(ctx->device);
     hk::GdnArgs a{q, k, v, q_tok, k_tok, v_tok, heads / k_heads, g, beta, (long)heads, cu, initial_state,
                   final_state, o, o_tok, heads, n_tokens, ctx->fault_dev, init_rows, final_rows};
+    // (the split form reads q and k after it has written part of o: o in their place stays with one kernel)
+    if (mfma && dtype == HK_F32 && delta_split_takes(n_seqs, n_tokens, heads) && o != q && o != k) {
+        if (void* scratch = split_scratch_for(ctx, hk_delta_split_bytes(n_tokens, n_seqs, heads), may_alloc)) {
+            const int rc = hk_launch_delta_split(&a, n_seqs, n_tokens / 64 + n_seqs, scratch, ctx->stream);
+            return rc ? hk_fail(ctx, rc, "gated delta launch failed") : HK_OK;
+        }
+    }
     int rc = mfma ? hk_launch_gated_delta_chunked(dtype, &a, n_seqs, ctx->stream)
                   : hk_launch_delta_gen(dtype, &a, dk, dv, n_seqs, ctx->stream);
     return rc ? hk_fail(ctx, rc, "gated delta launch failed") : HK_OK;
@@ -623,7 +645,7 @@ extern "C" int hk_gated_delta_chunked(hk_ctx* ctx, int dtype, const void* q, lon
                                       int n_seqs, int n_tokens, int heads, int k_heads, int dk, int dv,
                                       const float* initial_state, float* final_state, void* o, long o_tok) {
     return hk_gated_delta_chunked_rows(ctx, dtype, q, q_tok, k, k_tok, v, v_tok, g, beta, cu, n_seqs, n_tokens, heads,
-                                       k_heads, dk, dv, initial_state, final_state, o, o_tok, nullptr, nullptr);
+                                       k_heads, dk, dv, initial_state, final_state, o, o_tok, nullptr, nullptr, true);
 }
 
 int hk_gdn_prep_rows(hk_ctx* ctx, int dtype, const void* mixed, long mixed_tok, const float* conv_w, int conv_k,

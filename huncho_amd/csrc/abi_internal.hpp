@@ -35,6 +35,7 @@ constexpr size_t kSplitScratchMax = 512u << 20;
 bool hk_split_scratch_reserve(hk_ctx* ctx, size_t bytes);
 // Bytes for the chunks of n_tokens tokens in n_seqs rows.
 size_t hk_gdn_split_bytes(int n_tokens, int n_seqs, int heads);
+size_t hk_delta_split_bytes(int n_tokens, int n_seqs, int heads);
 
 int hk_fail(hk_ctx* ctx, int code, const char* fmt, ...);
 int hk_check_hip(hk_ctx* ctx, hipError_t e, const char* what);

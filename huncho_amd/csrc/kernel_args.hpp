@@ -83,6 +83,9 @@ struct GdnFusedArgs {
 // Scratch bytes of one (64-token chunk, head) of the fused layer for few, long rows (gdn16_split.hip)
 constexpr int HK_GDN_SPLIT_SLOT = 114688;
 
+// Scratch bytes of one (64-token chunk, head) of the fp32 delta rule for few rows (delta_rule_split.hip)
+constexpr int HK_DELTA_SPLIT_SLOT = 4 * (2 * 64 * 64 + 4 * 64 + 64 * 128 + 128 * 128);
+
 struct KvArgs {
     const void* q_in;
     long q_in_tok, q_in_head;
@@ -342,6 +345,7 @@ int hk_launch_seq_lens(const int* cu, int n, int* out, hipStream_t st);
 int hk_launch_token_seq_pos(const int* cu, const int* ctxl, int n_seqs, int n_tokens, int* out, int* fault,
                             hipStream_t st);
 int hk_launch_readout(int dtype, const hk::ReadoutArgs* a, hipStream_t st);
+int hk_launch_delta_split(const hk::GdnArgs* a, int n_seqs, int n_slots, void* scratch, hipStream_t stream);
 int hk_launch_gdn16_split(int dtype16, const hk::GdnArgs* a, const hk::GdnFusedArgs* fa, int n_seqs, int n_slots,
                           void* scratch, hipStream_t stream);
 int hk_launch_gemm(int dtype16, int epi, const hk::GemmArgs* a, hipStream_t stream);

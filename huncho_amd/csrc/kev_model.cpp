@@ -233,8 +233,10 @@ extern "C" int hk_kev_model_create(hk_ctx* ctx, int dtype, const hk_kev_config* 
     // DeltaNet layers, at most half of the limit, so that no forward allocates (batches that do not fit
     // run the layer without it)
     if (dtype != HK_F32 && (c.head_dim == 128 || c.head_dim == 256)) hk_split_scratch_reserve(ctx, hk_attn_split_bytes(c.head_dim));
-    if (dtype != HK_F32 && c.conv_k == 4 && c.lin_key_dim == 128 && c.lin_v_dim == 128) {
-        const size_t want = hk_gdn_split_bytes(4 * (c.max_context < 65536 ? c.max_context : 65536), 4, c.lin_n_v_heads);
+    if ((dtype == HK_F32 || c.conv_k == 4) && c.lin_key_dim == 128 && c.lin_v_dim == 128) {
+        const int tokens = 4 * (c.max_context < 65536 ? c.max_context : 65536);
+        const size_t want = dtype == HK_F32 ? hk_delta_split_bytes(tokens, 4, c.lin_n_v_heads)
+                                            : hk_gdn_split_bytes(tokens, 4, c.lin_n_v_heads);
         hk_split_scratch_reserve(ctx, want < kSplitScratchMax / 2 ? want : kSplitScratchMax / 2);
     }
     hipStreamSynchronize(nullptr);  // the weight copies, on the null stream, are complete before the
@@ -491,7 +493,7 @@ int kev_forward_impl(hk_kev_model* m, const int32_t* ids, const int32_t* cu_dev,
                 RUN(hk_gated_delta_chunked_rows(ctx, dt, b.q, (long)Hk * dk, b.k, (long)Hk * dk, b.v, (long)Hv * dv,
                                                 b.g, b.beta, cu_dev, n_seqs, n, Hv, Hk, dk, dv, nullptr, nullptr, b.o,
                                                 (long)Hv * dv, view ? view->init_rows[gi] : nullptr,
-                                                view ? view->final_rows[gi] : nullptr));
+                                                view ? view->final_rows[gi] : nullptr, false));
                 RUN(hk_gated_rms_norm(ctx, dt, b.o, (char*)b.big + (size_t)m->conv_dim * e, rows, Hv, L.norm_w, c.eps,
                                       n * Hv, dv, b.o));
             }

@@ -75,7 +75,10 @@ typedef struct {
 int hk_ctx_create(int device_ordinal, hk_ctx** out);
 int hk_ctx_destroy(hk_ctx* ctx);
 /* Work is ordered on this hipStream_t from now on (NULL: HIP's null stream). A new
- * context uses its own default-priority stream, returned by hk_ctx_own_stream. */
+ * context uses its own default-priority stream, returned by hk_ctx_own_stream. The scratch that
+ * the context keeps for batches of few, long rows (at most 512 MiB, grown by per-op calls and at
+ * model creation, freed with the context) follows it: the first use on the new stream waits for
+ * the old stream's last. The stream that the context leaves must still exist at this call. */
 int hk_ctx_set_stream(hk_ctx* ctx, void* hip_stream);
 void* hk_ctx_stream(hk_ctx* ctx);
 void* hk_ctx_own_stream(hk_ctx* ctx);
@@ -87,12 +90,12 @@ int hk_ctx_take_faults(hk_ctx* ctx, int* faults_out);
 int hk_device_count(int* out);
 const char* hk_version(void);
 
-/* ---- dense projections (hipBLASLt) ------------------------------------------------------------
+/* ---- dense projections ------------------------------------------------------------
  * The context's GEMM algorithm per shape is a deterministic function of the shape by default:
- * a solution pinned for the shape at build time, else hipBLASLt's heuristic first choice. The
- * GEMM handle and workspace are created with the first model on the context, so a forward
+ * the library's own few-row kernel where a 16-bit product has few rows, else a solution pinned for
+ * the shape at build time, else hipBLASLt's heuristic first choice. The GEMM handle and workspace are created with the first model on the context, so a forward
  * never allocates, times or synchronises. hk_ctx_set_gemm_autotune(ctx, 1) makes shapes first
- * seen afterwards time every supported solution instead (allocates scratch and synchronises
+ * seen afterwards time every supported hipBLASLt solution instead (allocates scratch and synchronises
  * on that first use; the choice then follows the device's timing). No reference counterpart:
  * candle's Linear (qwen3_5.rs:306-515) calls its BLAS with the library's own choice.
  * hk_ctx_gemm_plans writes one line per cached plan ("dtype= out= n= in= ... index= source")

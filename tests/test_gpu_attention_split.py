@@ -67,8 +67,8 @@ def run(ctx, q_lens, ctx_lens, hq, hkv, d, page, dtype, gate, seed, spare=0):
 @pytest.mark.parametrize("gate", [False, True])
 @pytest.mark.parametrize("q_lens,ctx_lens,hq,hkv,d,page", [
     ([1], [1024], 16, 8, 128, 16), ([30, 20, 40], [2700, 2701, 2751], 16, 8, 128, 16), ([1], [4097], 8, 8, 128, 64),
-    ([64, 3], [2048, 10], 16, 8, 128, 16), ([65], [1985], 16, 8, 128, 32), ([1500], [1500], 16, 8, 128, 16),
-    ([200, 1, 700], [900, 3000, 700], 16, 2, 128, 16), ([33], [3000], 8, 2, 256, 16), ([700], [1300], 16, 4, 256, 16)])
+    ([64, 3], [2048, 10], 16, 8, 128, 16), ([65], [1985], 16, 8, 128, 32), ([300], [1500], 16, 8, 128, 16),
+    ([200, 1, 500], [900, 3000, 700], 16, 2, 128, 16), ([33], [3000], 8, 2, 256, 16), ([200], [1300], 16, 4, 256, 16)])
 def test_split_matches_float64(ctx, dtype, gate, q_lens, ctx_lens, hq, hkv, d, page):
     _, e = run(ctx, q_lens, ctx_lens, hq, hkv, d, page, dtype, gate, sum(q_lens) + sum(ctx_lens))
     assert e < TOL[dtype], e
@@ -80,6 +80,21 @@ def test_short_context_under_a_wide_table(ctx):
     a, _ = run(ctx, [20], [150], 16, 8, 128, 16, torch.bfloat16, True, 5)
     b, e = run(ctx, [20], [150], 16, 8, 128, 16, torch.bfloat16, True, 5, spare=500)
     assert torch.equal(a, b) and e < TOL[torch.bfloat16]
+
+
+def test_a_fresh_row_keeps_its_bits(ctx):
+    """A row without cached tokens is not split: alone it gives the bits that it has in a large batch."""
+    a, _ = run(ctx, [1100], [1100], 16, 8, 128, 16, torch.bfloat16, True, 7)
+    g = torch.Generator(device="cuda").manual_seed(7)  # the same row first among 40
+    r = lambda *s: torch.randn(s, generator=g, device="cuda").to(torch.bfloat16)
+    need = (1100 + 15) // 16
+    kp, vp, qg = r(need, 8, 16, 128), r(need, 8, 16, 128), r(1100, 16, 256)
+    bt = torch.from_numpy(np.random.default_rng(7).permutation(need).astype(np.int32)).cuda().view(1, -1).repeat(40, 1)
+    cu = torch.arange(0, 40 * 1100 + 1, 1100, dtype=torch.int32, device="cuda")
+    q = qg.repeat(40, 1, 1)
+    o = paged_prefill_attention(ctx, q[:, :, :128], kp, vp, bt, cu, torch.full((40,), 1100, dtype=torch.int32, device="cuda"),
+                                1100, gate=q[:, :, 128:])
+    assert torch.equal(a, o[:1100]) and torch.equal(a, o[-1100:])
 
 
 def test_nan_and_infinite_scores(ctx):
