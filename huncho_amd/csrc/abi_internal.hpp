@@ -70,6 +70,11 @@ size_t hk_attn_split_bytes(int head_dim);
 int hk_gemm_xwt_pair(hk_ctx* ctx, int dtype, int n, int in, const void* x, long ldx, int out, const void* w, void* y,
                      int out2, const void* w2, void* y2);
 
+// y [n][inter] = gelu(x Wg^T) * (x Wu^T) of the stacked weight [Wg | Wu] [2 inter][in], each product rounded to
+// the dtype first, in one launch for few rows; false (nothing launched) where the projection and the
+// GeGLU pass on their own are the way.
+bool hk_gemm_geglu_few_rows(hk_ctx* ctx, int dtype, int n, int inter, int in, const void* x, const void* w, void* y, int* rc);
+
 // hk_qk_norm_rope_kv_write with an optional per-token (sequence, position) table (int pairs,
 // hk_launch_token_seq_pos), which replaces the kernel's search of cu_seqlens
 int hk_qk_norm_rope_kv_write_impl(hk_ctx* ctx, int dtype, const void* q_in, long q_in_tok, long q_in_head,

@@ -414,8 +414,6 @@ __global__ __launch_bounds__(256) void layer_norm(LayerNormArgs a) {
     }
 }
 
-__device__ __forceinline__ float gelu_erf(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
-
 // y[t][i] = gelu(x[t][i]) * x[t][I + i], fp32 arithmetic; VEC: N elements per thread with
 // 16-byte accesses.
 template <typename T, bool VEC>

@@ -275,9 +275,14 @@ extern "C" int hk_bert_forward(hk_bert_model* m, const int32_t* ids, const int32
                  : 0);
         BRUN(hk_gemm_xwt(ctx, dt, n, H, H, b.att, H, L.wo, H, b.h, H, b.h, H, 1.0f, 1.0f));
         BRUN(hk_layer_norm(ctx, dt, b.h, H, L.mlp_norm, c.eps, n, H, b.x, H));
-        BRUN(hk_gemm_xwt(ctx, dt, n, 2 * I, H, b.x, H, L.wi, H, b.gi, 2 * I, nullptr, 0, 1.0f, 0.0f));
-        hk::GegluArgs ga{b.gi, 2L * I, n, I, b.act, (long)I};
-        BRUN(hk_launch_geglu(dt, &ga, ctx->stream) ? hk_fail(ctx, HK_ERR_DEVICE, "geglu launch") : 0);
+        int rc = HK_OK;
+        if (hk_gemm_geglu_few_rows(ctx, dt, n, I, H, b.x, L.wi, b.act, &rc)) {
+            BRUN(rc);
+        } else {
+            BRUN(hk_gemm_xwt(ctx, dt, n, 2 * I, H, b.x, H, L.wi, H, b.gi, 2 * I, nullptr, 0, 1.0f, 0.0f));
+            hk::GegluArgs ga{b.gi, 2L * I, n, I, b.act, (long)I};
+            BRUN(hk_launch_geglu(dt, &ga, ctx->stream) ? hk_fail(ctx, HK_ERR_DEVICE, "geglu launch") : 0);
+        }
         BRUN(hk_gemm_xwt(ctx, dt, n, H, I, b.act, I, L.wo2, I, b.h, H, b.h, H, 1.0f, 1.0f));
     }
     void* fin = hidden_out ? hidden_out : b.x;

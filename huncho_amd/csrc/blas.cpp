@@ -209,8 +209,9 @@ int hk_gemm_xwt(hk_ctx* ctx, int dtype, int n, int out, int in, const void* x, l
 static bool few_rows_takes(int dtype, int epi, const hk::GemmArgs& a) {
     if (dtype != HK_BF16 && dtype != HK_F16) return false;
     const long ldc = a.c ? a.ldc : 0;
-    if (a.K <= 0 || a.K % 64 || a.N <= 0 || a.N % (epi == hk::EPI_SWIGLU ? 32 : 8) || a.N2 % 8 || a.ldx % 8 || a.ldw % 8 ||
-        a.ldy % 8 || ldc % 8 || a.ldy2 % 8 || a.ldx >= 1 << 22 || a.ldw >= 1 << 22)
+    const bool glu = epi == hk::EPI_SWIGLU || epi == hk::EPI_GEGLU;
+    if (a.K <= 0 || a.K % 64 || a.N <= 0 || a.N % (glu ? 32 : 8) || a.N2 % 8 || a.ldx % 8 || a.ldw % 8 || a.ldy % 8 ||
+        ldc % 8 || a.ldy2 % 8 || a.ldx >= 1 << 22 || a.ldw >= 1 << 22)
         return false;
     return (((uintptr_t)a.x | (uintptr_t)a.w | (uintptr_t)a.c | (uintptr_t)a.y | (uintptr_t)a.w2 | (uintptr_t)a.y2) & 15) == 0;
 }
@@ -235,6 +236,20 @@ int hk_gemm_xwt_pair(hk_ctx* ctx, int dtype, int n, int in, const void* x, long 
                                                                            : HK_OK;
     if (int rc = hk_gemm_xwt(ctx, dtype, n, out, in, x, ldx, w, in, y, out, nullptr, 0, 1.0f, 0.0f)) return rc;
     return hk_gemm_xwt(ctx, dtype, n, out2, in, x, ldx, w2, in, y2, out2, nullptr, 0, 1.0f, 0.0f);
+}
+
+// The encoder's GeGLU in the projection's epilogue, wherever the few-row kernel would take the projection: one
+// launch and one pass over 2 inter columns less (encoder of 22 layers, 653 rows: 1256 -> 1234 us; two runs
+// of one side differ by 0.2 %). In the library's range the pass on its own is the faster one (erf in the epilogue
+// of large tiles leaves the matrix cores idle).
+bool hk_gemm_geglu_few_rows(hk_ctx* ctx, int dtype, int n, int inter, int in, const void* x, const void* w, void* y, int* rc) {
+    const hk::GemmArgs a{x, w, nullptr, y, in, in, 0, inter, n, 2 * inter, in, nullptr, nullptr, 0, 0};
+    if (n <= 0 || !ctx->blas || ctx->blas->autotune || 4L * inter * in >= 1L << 31 || !few_rows_takes(dtype, hk::EPI_GEGLU, a) ||
+        !few_rows_wins(hk::EPI_GEGLU, a))
+        return false;
+    *rc = hk_launch_gemm_few_rows(dtype, hk::EPI_GEGLU, &a, ctx->stream) ? hk_fail(ctx, HK_ERR_DEVICE, "gemm launch failed")
+                                                                         : HK_OK;
+    return true;
 }
 
 int hk_gemm_xwt_cd(hk_ctx* ctx, int dtype, int cd_dtype, int n, int out, int in, const void* x, long ldx,

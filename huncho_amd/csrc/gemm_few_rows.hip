@@ -18,6 +18,8 @@
 //   169 rows, residual 1024 x 3584      104 -> 11.2      2704 rows  99.4 -> 38.7
 //   169 rows, store 8192 x 1024        32.7 -> 9.5        (library 13.6)
 //    64 rows, store 2304 x 768         19.2 -> 4.8        (library 7.5)
+//   653 rows, GeGLU 2304 x 768: a forward of 22 such layers 1256 -> 1234 against store and the pass over
+//                              its rows (the same bits)
 // U steps of 64 share a barrier where a wave has few products per step: 32 x 32 tiles over K 3584 took
 // 15.7 us with a barrier per step, at any depth of the ring, and 11.2 with one per 4.
 //
@@ -73,7 +75,7 @@ template <> __device__ __forceinline__ f32x4 mma16x32<f16>(f16x8 a, f16x8 b, f32
 template <typename T, int EPI, int NB, int MB, int ST, int U>
 __global__ __launch_bounds__(NTHREADS, 2) void gemm_few_rows(GemmArgs a) {
     typedef typename Mma16<T>::v8 v8;
-    constexpr bool SWI = EPI == EPI_SWIGLU, RES = EPI == EPI_RESIDUAL || EPI == EPI_RESIDUAL_F32;
+    constexpr bool GEGLU = EPI == EPI_GEGLU, SWI = EPI == EPI_SWIGLU || GEGLU, RES = EPI == EPI_RESIDUAL || EPI == EPI_RESIDUAL_F32;
     typedef typename std::conditional<EPI == EPI_RESIDUAL_F32, float, T>::type TY;  // rows of c and y
     typedef TY y4 __attribute__((ext_vector_type(4)));
     constexpr int STAGE = (NB + MB) * BLK_BYTES, CPW = NB + MB;  // copies per wave and stage
@@ -113,7 +115,11 @@ __global__ __launch_bounds__(NTHREADS, 2) void gemm_few_rows(GemmArgs a) {
 
     const int crow = lane >> 3, cpc = lane & 7;
     const int lc0 = cpc ^ (crow >> 1), lc1 = cpc ^ (4 + (crow >> 1));
-    const i32x4_t wrs = buffer_rsrc((const T*)a.w + (long)n0 * a.ldw, (unsigned)(min(32 * NB, a.N - n0) * a.ldw * 2));
+    // GeGLU: the weight holds all gate rows, then all up rows, and the tile's 32-row block c takes gate rows
+    // n0 / 2 + 16 c .. + 15 (copies of waves 0 and 1) and their up rows N / 2 further on (waves 2 and 3): the
+    // block layout that SwiGLU weights are stored in
+    const i32x4_t wrs = GEGLU ? buffer_rsrc(a.w, (unsigned)(a.N * a.ldw * 2))
+                              : buffer_rsrc((const T*)a.w + (long)n0 * a.ldw, (unsigned)(min(32 * NB, a.N - n0) * a.ldw * 2));
     const i32x4_t xrs = buffer_rsrc((const T*)a.x + (long)m0 * a.ldx, (unsigned)(min(32 * MB, a.M - m0) * a.ldx * 2));
     // copy c of a stage: 8 rows, odd copies with the swizzle of rows 8 .. 15; wave w issues copies w, w + 4,
     // .. of both operands, all of w's parity
@@ -125,7 +131,10 @@ __global__ __launch_bounds__(NTHREADS, 2) void gemm_few_rows(GemmArgs a) {
     auto load_step = [&](int t) {
         const unsigned dst = lds0 + (unsigned)(t % ST) * STAGE, so = (unsigned)t * ROW_BYTES;
 #pragma unroll
-        for (int c = 0; c < NB; ++c) buf_copy_x4(wrs, wv, so + (4 * c + wave) * w8, dst + (4 * c + wave) * (8 * ROW_BYTES));
+        for (int c = 0; c < NB; ++c) {
+            const unsigned wo = GEGLU ? (unsigned)(n0 / 16 + 2 * c + (wave & 1) + (wave >> 1) * (a.N / 16)) * w8 : (4 * c + wave) * w8;
+            buf_copy_x4(wrs, wv, so + wo, dst + (4 * c + wave) * (8 * ROW_BYTES));
+        }
 #pragma unroll
         for (int c = 0; c < MB; ++c)
             buf_copy_x4(xrs, xv, so + (4 * c + wave) * x8, dst + (4 * (NB + c) + wave) * (8 * ROW_BYTES));
@@ -194,9 +203,10 @@ __global__ __launch_bounds__(NTHREADS, 2) void gemm_few_rows(GemmArgs a) {
                 for (int jj = 0; jj < 2; ++jj) {
                     y4 o;
 #pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        o[r] = from_f<TY>(silu_f<T>(to_f(from_f<T>(acc[i][jb][4 * jj + r]))) *
-                                          to_f(from_f<T>(acc[i][jb][4 * (jj + 2) + r])));
+                    for (int r = 0; r < 4; ++r) {
+                        const float gv = to_f(from_f<T>(acc[i][jb][4 * jj + r]));
+                        o[r] = from_f<TY>((GEGLU ? gelu_erf(gv) : silu_f<T>(gv)) * to_f(from_f<T>(acc[i][jb][4 * (jj + 2) + r])));
+                    }
                     if (m < a.M && nb < a.N) *(y4*)((TY*)a.y + (long)m * a.ldy + nb / 2 + 8 * jj + 4 * g) = o;
                 }
             } else {
@@ -233,7 +243,7 @@ long n_tiles(const hk::GemmArgs* a, const Tile& t) {
 int best_tile(int epi, const hk::GemmArgs* a, float* cost) {
     int best = -1;
     for (int i = 0; i < kNumTiles; ++i) {
-        if (epi == hk::EPI_SWIGLU && (kTiles[i].nb % 2 || kTiles[i].mb % 2)) continue;  // four waves' 32 x 32 blocks
+        if ((epi == hk::EPI_SWIGLU || epi == hk::EPI_GEGLU) && (kTiles[i].nb % 2 || kTiles[i].mb % 2)) continue;  // four waves' 32 x 32 blocks
         const Tile& k = kTiles[i];
         const long n = n_tiles(a, k);
         const float c = n <= 256 ? k.first : k.round > 0.0f ? k.round * (float)((n + 511) / 512) : k.first + k.slope * (float)(n - 256);
@@ -249,7 +259,7 @@ int best_tile(int epi, const hk::GemmArgs* a, float* cost) {
 template <typename T, int EPI, int I, int ST, int U>
 static int launch_one(const hk::GemmArgs* a, hipStream_t stream) {
     constexpr int NB = kTiles[I].nb, MB = kTiles[I].mb;
-    if constexpr (EPI == hk::EPI_SWIGLU && (NB % 2 || MB % 2)) {
+    if constexpr ((EPI == hk::EPI_SWIGLU || EPI == hk::EPI_GEGLU) && (NB % 2 || MB % 2)) {
         return HK_ERR_DEVICE;  // best_tile does not choose it
     } else {
         constexpr int lds = ST * (NB + MB) * hk::gemm_few::BLK_BYTES;
@@ -288,6 +298,7 @@ static int launch_type(int epi, const hk::GemmArgs* a, hipStream_t stream) {
         case hk::EPI_RESIDUAL: return launch_epi<T, hk::EPI_RESIDUAL>(a, stream);
         case hk::EPI_RESIDUAL_F32: return launch_epi<T, hk::EPI_RESIDUAL_F32>(a, stream);
         case hk::EPI_SWIGLU: return launch_epi<T, hk::EPI_SWIGLU>(a, stream);
+        case hk::EPI_GEGLU: return launch_epi<T, hk::EPI_GEGLU>(a, stream);
         default: return launch_epi<T, hk::EPI_STORE>(a, stream);
     }
 }
@@ -299,7 +310,7 @@ extern "C" float hk_gemm_few_rows_cost(int epi, const hk::GemmArgs* a) {
     return cost;
 }
 
-// dtype16: 1 = bf16, 2 = fp16. The caller has checked: N and N2 % 8 == 0 (SwiGLU: N % 32), K % 64 == 0,
+// dtype16: 1 = bf16, 2 = fp16. The caller has checked: N and N2 % 8 == 0 (SwiGLU, GeGLU: N % 32), K % 64 == 0,
 // 16-byte aligned rows (ld % 8 == 0) and row strides below 2^22 elements (32-bit copy offsets).
 extern "C" int hk_launch_gemm_few_rows(int dtype16, int epi, const hk::GemmArgs* a, hipStream_t stream) {
     if (a->M == 0) return HK_OK;

@@ -302,8 +302,9 @@ struct ReadoutArgs {
 };
 
 // Dense projection Y = X W^T with a fused epilogue (gemm.hip; gemm_few_rows.hip for few rows, which
-// also has EPI_RESIDUAL_F32: fp32 rows of c and y, the fp32 residual stream).
-enum { EPI_STORE = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2, EPI_RESIDUAL_F32 = 3 };
+// also has EPI_RESIDUAL_F32: fp32 rows of c and y, the fp32 residual stream; and EPI_GEGLU: y =
+// T(gelu(T(g)) * T(u)) of w's first and second N / 2 rows).
+enum { EPI_STORE = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2, EPI_RESIDUAL_F32 = 3, EPI_GEGLU = 4 };
 struct GemmArgs {
     const void* x;  // [M][K], row stride ldx
     const void* w;  // [N][K], row stride ldw

@@ -73,3 +73,25 @@ def test_rows_do_not_depend_on_the_batch(ctx, dtype, epi, n, k):
     whole = linear(ctx, x, w, epi, c, cols)  # gemm.hip
     for rows in (1, 40, 100, 169, 300, 600, 1200):
         assert torch.equal(linear(ctx, x[:rows], w, epi, c[:rows] if epi == 1 else None, cols), whole[:rows]), rows
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hidden,heads,inter", [(768, 12, 1152), (256, 4, 176)])
+def test_encoder_rows_do_not_depend_on_the_batch(ctx, dtype, hidden, heads, inter):
+    """The encoder's few-row path (its GeGLU projection in one launch) gives a row the bits that it has
+    in a batch of many rows, which runs the projection and the GeGLU pass on their own. 176 gate columns
+    leave a part of a tile."""
+    import numpy as np
+
+    from huncho_amd.laya import LayaModel, LayaShape, synthetic_weights
+
+    shape = LayaShape(hidden=hidden, n_layers=3, n_heads=heads, intermediate=inter, vocab=500, max_context=512, n_out=2)
+    model = LayaModel(ctx, shape, synthetic_weights(shape, 3, std=0.05), dtype)
+    rng = np.random.default_rng(1)
+    rows = [rng.integers(0, 500, n).tolist() for n in [70, 1, 200] + [500] * 24]
+    many, hm = model.forward_batch(rows, want_hidden=True)
+    for n in (1, 2, 3):
+        few, hf = model.forward_batch(rows[:n], want_hidden=True)
+        assert all(np.array_equal(a, b) for a, b in zip(hf, hm[:n]))
+        assert np.array_equal(few, many[:n])
+    model.close()
