@@ -210,109 +210,6 @@ __device__ __forceinline__ typename M16<T>::v4 ld_a4(const float* Am, int r, int
                : typename M16<T>::v4{(T)x[0], (T)x[1], (T)x[2], (T)x[3]};
 }
 
-// P0 of the fused layer: the conv, SiLU and l2norm of chunk rows c0 .. c0 + 63 of q, k and v (the raw
-// in_proj rows of the sequence that starts at token t0) into the LDS tiles.
-template <typename T>
-__device__ __forceinline__ void fused_rows(const GdnFusedArgs& fa, int t0, int Tn, int c0, int h, int kh, const T* hist,
-                                           int wave, int q4, int j, f16* Qs, f16* Ks, f16* Vs) {
-    typedef f16 CT;
-    typedef typename M16<CT>::v8 v8;
-    typedef typename M16<T>::v8 tv8;
-    typedef typename M16<T>::v2 tv2;
-    // 16 lane groups (4 per wave) x 4 rows of each of q, k and v: group G = 4 wave + q4
-    // takes chunk rows 4 G .. 4 G + 3 of every tensor, so all four waves share the conv,
-    // SiLU and l2norm evenly. Each tensor's 4 conv outputs come from a 7-row window of raw
-    // conv inputs (sequence positions c0 + 4 G - 3 ..). Positions past the sequence end
-    // are loaded clamped: they only reach rows past the end, whose beta is 0 and whose
-    // outputs are not stored. Positions before the start are the conv history or 0.
-    const int r0 = 4 * (4 * wave + q4);
-    auto tcol = [&](int tsr) {  // mixed column of this lane's channels in tensor tsr
-        return (tsr == 2 ? 2 * (long)fa.Hk * 128 + (long)h * 128 : (long)tsr * fa.Hk * 128 + (long)kh * 128) +
-               8 * j;
-    };
-    // all three windows are loaded before the first conv, so the chunk waits for one
-    // memory round trip
-    // Addresses: a wave-uniform base per tensor (this sequence's first row, the head's
-    // columns) plus one 32-bit byte offset per row shared by the three tensors (the host
-    // keeps n_tokens * mixed_tok * sizeof(T) below 2^32 and the row stride below 2^24)
-    tv8 raw[3][7];
-    {
-        const char* const mb = (const char*)fa.mixed + (long)t0 * fa.mixed_tok * (long)sizeof(T);
-        const char* const base[3] = {mb + (long)kh * 128 * sizeof(T),
-                                     mb + ((long)fa.Hk + kh) * 128 * sizeof(T),
-                                     mb + (2L * fa.Hk + h) * 128 * sizeof(T)};
-        const unsigned row_b = (unsigned)(fa.mixed_tok * sizeof(T));
-#pragma unroll
-        for (int i = 0; i < 7; ++i) {
-            const int p = c0 + r0 - 3 + i;
-            const unsigned pc = (unsigned)(p < 0 ? 0 : (p >= Tn ? Tn - 1 : p));
-            const unsigned off = __umul24(pc, row_b) + 16u * j;
-#pragma unroll
-            for (int tsr = 0; tsr < 3; ++tsr) raw[tsr][i] = *(const tv8*)(base[tsr] + off);
-        }
-    }
-    if (c0 + r0 == 0) {  // windows start 3 positions before the sequence
-#pragma unroll
-        for (int tsr = 0; tsr < 3; ++tsr) {
-            if (hist) {
-                const T* hb = hist + tcol(tsr) * 3;
-#pragma unroll
-                for (int i = 0; i < 3; ++i)
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) raw[tsr][i][e] = hb[e * 3 + i];
-            } else {
-#pragma unroll
-                for (int i = 0; i < 3; ++i) raw[tsr][i] = tv8{};
-            }
-        }
-    }
-#pragma unroll
-    for (int tsr = 0; tsr < 3; ++tsr) {
-        const long mct = tcol(tsr);
-        CT* dst = tsr == 0 ? Qs : tsr == 1 ? Ks : Vs;
-        // taps (0, 1) and (2, 3) of each channel as 16-bit pairs (the weights are the
-        // model dtype's values, exact in T)
-        tv2 w01[8], w23[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const f32x4 w4 = *(const f32x4*)(fa.conv_w + (mct + e) * 4);
-            w01[e] = tv2{(T)w4[0], (T)w4[1]};
-            w23[e] = tv2{(T)w4[2], (T)w4[3]};
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float y[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float acc = dot2(w23[e], tv2{raw[tsr][i + 2][e], raw[tsr][i + 3][e]},
-                                       dot2_0(w01[e], tv2{raw[tsr][i][e], raw[tsr][i + 1][e]}));
-                y[e] = silu(acc);
-            }
-            // the conv output is stored in T (qwen3_5.rs:843), held exactly in CT
-            f16x2 o[4];
-            if (tsr < 2) {  // conv output stored in the activation dtype, then l2norm over
-                            // the head's 128 channels (16 lanes); q also takes the scale
-                tv2 p[4];
-#pragma unroll
-                for (int m = 0; m < 4; ++m) p[m] = tv2{(T)y[2 * m], (T)y[2 * m + 1]};
-                float ss = dot2_0(p[0], p[0]);
-#pragma unroll
-                for (int m = 1; m < 4; ++m) ss = dot2(p[m], p[m], ss);
-                ss = sum16(ss);
-                const float inv = fast_rsqrt(ss + 1e-6f) * (tsr == 0 ? fa.scale : 1.0f);
-                // the normalised q and k stay fp32 in the reference (l2norm returns
-                // fp32, qwen3_5.rs:204-210, 923-924): rounded only to the fp16 operand
-#pragma unroll
-                for (int m = 0; m < 4; ++m) o[m] = f16x2{(f16)(lo_f(p[m]) * inv), (f16)(hi_f(p[m]) * inv)};
-            } else {
-#pragma unroll
-                for (int m = 0; m < 4; ++m) o[m] = rnd_ct<T>(y[2 * m], y[2 * m + 1]);
-            }
-            *(v8*)(dst + el(r0 + i, 8 * j)) = __builtin_bit_cast(v8, o);
-        }
-    }
-}
-
 // P1's tiles of A = strict_lower(beta e^(G_t - G_s) k_t.k_s) in fp32 and Aqk = lower(e^(G_t - G_s) q_t.k_s).
 __device__ __forceinline__ void chunk_tiles(const f16* Qs, const f16* Ks, const float* Gs, const float* Bs, float* Am,
                                             f16* Aq, int wave, int q4, int j) {
@@ -510,7 +407,7 @@ __global__ __launch_bounds__(256, 2) void gdn_chunk16(GdnArgs a, GdnFusedArgs fa
         __syncthreads();
         // ---------------- P0: inputs -> LDS ----------------
         if (FUSED) {
-            fused_rows<T>(fa, t0, Tn, c0, h, kh, hist, wave, q4, j, Qs, Ks, Vs);
+#include "gdn16_rows.inc"
         } else {
             // 3 tensors x 64 rows x 16 chunks = 12 chunks per lane; 16 lanes per row
             tv8 x[12];
