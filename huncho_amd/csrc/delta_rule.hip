@@ -47,6 +47,9 @@ __global__ __launch_bounds__(256, 1) void gdn_chunk_f32(GdnArgs a) {
     }
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 5, col = lane & 31;
     const int dvc = wave * 32 + col;  // this lane's value column
+    const int kh = h / a.qk_rep;
+    const float* qg = (const float*)a.q + (long)kh * DK;
+    const float* kg = (const float*)a.k + (long)kh * DK;
     const float* vg = (const float*)a.v + (long)h * DV;
     float* og = (float*)a.o + (long)h * DV;
     // this sequence's state rows [H][dk][dv] (per-row pointer tables or contiguous arrays)
@@ -66,7 +69,10 @@ __global__ __launch_bounds__(256, 1) void gdn_chunk_f32(GdnArgs a) {
     for (int c0 = 0; c0 < T; c0 += CH) {
         const int Lc = min(CH, T - c0);
         __syncthreads();
-        load_chunk_f32(a, h, t0 + c0, Lc, Qc, Kc, Gs, Bs, tid, wave, lane);
+        {
+            const int t = t0 + c0;
+#include "delta_rule_load.inc"
+        }
         __syncthreads();
         chunk_matrices_f32(Qc, Kc, Gs, Bs, Am, Aq, wave, lane);
         __syncthreads();

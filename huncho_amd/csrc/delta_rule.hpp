@@ -107,34 +107,6 @@ constexpr int F_ASTR = CH + 4;  // fp32 row stride of A/T and Aqk
 constexpr int XSTR = 32 + 4;    // fp32 row stride of the inversion scratch
 constexpr size_t GDN_F32_LDS = sizeof(float) * (2 * CH * F_KSTR + 3 * CH * F_ASTR + 32 * XSTR + 2 * CH);
 
-// q and k of the Lc tokens from t on (zero rows past them), the inclusive scan of g and beta into LDS
-__device__ __forceinline__ void load_chunk_f32(const GdnArgs& a, int h, int t, int Lc, float* Qc, float* Kc, float* Gs,
-                                               float* Bs, int tid, int wave, int lane) {
-    const float* qg = (const float*)a.q + (long)(h / a.qk_rep) * DK;
-    const float* kg = (const float*)a.k + (long)(h / a.qk_rep) * DK;
-    // q, k chunk -> LDS (zero rows past the end); g, beta -> registers of wave 0
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        int idx = tid + 256 * i, r = idx >> 5, c4 = (idx & 31) * 4;
-        f32x4 qv = {0.f, 0.f, 0.f, 0.f}, kv = {0.f, 0.f, 0.f, 0.f};
-        if (r < Lc) {
-            qv = *(const f32x4*)(qg + (long)(t + r) * a.q_tok + c4);
-            kv = *(const f32x4*)(kg + (long)(t + r) * a.k_tok + c4);
-        }
-        *(f32x4*)(Qc + r * F_KSTR + c4) = qv;
-        *(f32x4*)(Kc + r * F_KSTR + c4) = kv;
-    }
-    if (wave == 0) {
-        float gv = 0.f, bv = 0.f;
-        if (lane < Lc) {
-            gv = a.g[(long)(t + lane) * a.gb_tok + h];
-            bv = a.beta[(long)(t + lane) * a.gb_tok + h];
-        }
-        Gs[lane] = wave_incl_scan(gv, lane);
-        Bs[lane] = bv;
-    }
-}
-
 // A and Aqk of a chunk [64][F_ASTR] from its q and k tiles
 __device__ __forceinline__ void chunk_matrices_f32(const float* Qc, const float* Kc, const float* Gs, const float* Bs, float* Am,
                                                    float* Aq, int wave, int lane) {

@@ -71,7 +71,12 @@ __global__ __launch_bounds__(256, 1) void delta_split_prep(GdnArgs a, int n_seqs
     int c0, t0, Tn;
     if (!find_chunk(a, n_seqs, cid, c0, t0, Tn)) return;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    load_chunk_f32(a, h, t0 + c0, min(CH, Tn - c0), Qc, Kc, Gs, Bs, tid, wave, lane);
+    {
+        const int t = t0 + c0, Lc = min(CH, Tn - c0);
+        const float* qg = (const float*)a.q + (long)(h / a.qk_rep) * DK;
+        const float* kg = (const float*)a.k + (long)(h / a.qk_rep) * DK;
+#include "delta_rule_load.inc"
+    }
     __syncthreads();
     chunk_matrices_f32(Qc, Kc, Gs, Bs, Am, Aq, wave, lane);
     __syncthreads();
