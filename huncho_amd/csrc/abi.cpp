@@ -477,24 +477,35 @@ extern "C" int hk_paged_kv_write(hk_ctx* ctx, int dtype, const void* k, const vo
                                          head_dim, nullptr, 0, 0, k_pool, v_pool, nullptr);
 }
 
-// Ranges of a q-block's key tiles for a batch that leaves most of the chip idle (1: not split): ranges of
-// 4 tiles or more, at most kAttnParts workgroups and the 32 ranges that attn_combine takes. Only for
-// suffixes, contexts of 1,024 tokens or more and at least four times as long as the rows: the sums of
-// split rows round differently, and a prefix computed alone keeps the bits that it has in a large batch.
-// There, where the estimates (us, 128-wide heads) favour it by 5 %: a pair of q-blocks runs its tiles at
-// 1.2 us one after another; a range pays 1.25 us a tile (1.75 with two workgroups per CU), and its parts
-// are written and read back. Measured, 16 / 8 heads, unsplit against split, rows x new tokens / context:
-//   1 x 30 / 1024 24.3 12.8, / 2700 54.8 13.5; 5 x 30 / 2700 55.7 23.1; 16 x 30 / 1024 26.3 26.8 (not
-//   split), / 4096 81.0 56.7; 4 x 128 / 2048 86.1 28.5
-static const int kAttnParts = 512;
-static int attn_splits(long blocks, long pairs, int tiles, int pair_tiles, bool paired) {
-    if (pairs >= 256 || blocks > kAttnParts / 2) return 1;
-    const int by_tiles = (tiles + 3) / 4, room = (int)(kAttnParts / blocks);
-    const int n = std::min(std::min(by_tiles, room), 32);
+// Ranges of a q-block of `tiles` key tiles in a batch that leaves most of the chip idle (1: not split): ranges
+// of 4 tiles or more, at most kAttnParts workgroups and the 32 ranges that attn_combine takes. Where the
+// estimates (us, 128-wide heads) favour it by 5 %: a pair of q-blocks runs its tiles at 1.2 us one after
+// another; a range pays 1.25 us a tile (1.75 with two workgroups per CU), and its parts are written and
+// read back. Measured, bf16, 16 / 8 heads, unsplit against split, rows x new tokens / context:
+//   1 x 30 / 1030 25.6 12.8, / 2700 54.6 13.1; 5 x 30 / 2700 55.0 19.1; 12 x 24 / 2524 51.2 27.2; 16 x 30 /
+//   1054 25.6 (not split), / 4096 78.0 43.6; 4 x 128 / 2048 87.4 26.8; 2 x 128 / 4128 168 26.7
+static int attn_splits(long blocks, int tiles, int pair_tiles, bool paired) {
+    const int n = std::min(std::min((tiles + 3) / 4, (int)(kAttnParts / blocks)), 32);
     const int per = (tiles + n - 1) / n;
     const float whole = 5.0f + 1.18f * pair_tiles + (paired ? 7.0f : 0.0f);
     const float split = 11.0f + per * (blocks * n > 256 ? 1.75f : 1.25f) + 0.0145f * (float)(blocks * n);
     return n > 1 && split < 0.95f * whole ? n : 1;
+}
+// The least number of key tiles from which a row of the batch is split (0: none is), and the most ranges of a
+// row of max_tiles tiles. Only suffixes, contexts of 16 tiles (1,024 tokens) or more and at least four times
+// as long as the row: the sums of split rows round differently, and a prefix computed alone keeps the bits
+// that it has in a large batch. Which rows those are the kernel decides, row by row; a row's ranges depend on
+// its own lengths, the number of rows and max_q_len, not on max_tiles.
+static int attn_split_from(long blocks, long pairs, int n_qblocks, int pos_per_block, int max_tiles, int* n_split) {
+    if (pairs >= 256 || blocks > kAttnParts / 2) return 0;
+    for (int t = 16; t <= std::min(max_tiles, 64); ++t) {  // (past 64 tiles it no longer depends on them)
+        // a pair's two blocks lie (n_qblocks - 1) x pos_per_block keys apart in all
+        const int pair_tiles = n_qblocks == 1 ? t : 2 * t - (n_qblocks - 1) * pos_per_block / 64;
+        if (attn_splits(blocks, t, pair_tiles, n_qblocks > 1) == 1) continue;
+        *n_split = std::min(std::min((max_tiles + 3) / 4, (int)(kAttnParts / blocks)), 32);
+        return t;
+    }
+    return 0;
 }
 size_t hk_attn_split_bytes(int head_dim) { return (size_t)kAttnParts * 128 * (head_dim + 2) * sizeof(float); }
 
@@ -556,16 +567,15 @@ int hk_paged_prefill_attention_impl(hk_ctx* ctx, int dtype, const void* q, long 
         const long most = (long)bt_stride << shift, keys = max_ctx > 0 && max_ctx < most ? max_ctx : most;
         const int tiles = (int)((keys + 63) / 64 < (1 << 20) ? (keys + 63) / 64 : 1 << 20);
         const long rows = (long)kv_heads * n_seqs;
-        // a pair's two blocks lie (n_qblocks - 1) x pos_per_block keys apart in all
-        const int pair_tiles = n_qblocks == 1 ? tiles : 2 * tiles - (n_qblocks - 1) * pos_per_block / 64;
-        const int n = tiles < 16 || keys / 4 < max_q_len
-                          ? 1
-                          : attn_splits(rows * n_qblocks, rows * ((n_qblocks + 1) / 2), tiles, pair_tiles, n_qblocks > 1);
+        int n = 1;
+        const int from = keys / 4 < max_q_len ? 0
+                                              : attn_split_from(rows * n_qblocks, rows * ((n_qblocks + 1) / 2), n_qblocks,
+                                                                pos_per_block, tiles, &n);
         const size_t bytes = (size_t)(rows * n_qblocks * n) * 128 * (head_dim + 2) * sizeof(float);
-        if (n > 1) {
+        if (from) {
             if (void* scratch = split_scratch_for(ctx, bytes, may_alloc)) {
                 a.n_split = n;
-                a.split_tiles = 4;
+                a.split_from = from;
                 a.n_qblocks = n_qblocks;
                 a.part = (float*)scratch;
                 a.part_ml = a.part + (size_t)(rows * n_qblocks * n) * 128 * head_dim;

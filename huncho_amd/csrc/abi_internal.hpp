@@ -29,6 +29,7 @@ struct hk_ctx {
     hipEvent_t split_moved = nullptr;
     bool split_wait = false, split_wait_all = false;
 };
+constexpr int kAttnParts = 512;  // most parts of a key-split attention launch, of at most half as many q-blocks
 constexpr size_t kSplitScratchMax = 512u << 20;
 // Ensures `bytes` of scratch (rounded up to a power of two, at least 32 MiB); frees and reallocates a smaller one after waiting
 // for its users. false if bytes exceed the limit or the allocation fails.

@@ -85,10 +85,12 @@ __device__ __forceinline__ int swz(int r) { return 4 * (r & 3); }
 __device__ __forceinline__ int swzk(int r) { return (r & 7) | (((r >> 4) & 1) << 3); }
 __device__ __forceinline__ int lds_off_k(int r, int c) { return r * KV_ROW + 8 * (c ^ swzk(r)); }
 
-// Key-split launches: tiles per range of a q-block of nt tiles (nt: one range), and the first part of a
-// q-block. The same in the attention and the combining kernel.
-__device__ __forceinline__ int split_range(const AttnArgs& a, int nt) {
-    return min(nt, max(a.split_tiles, (nt + a.n_split - 1) / a.n_split));
+// Key-split launches: tiles per range of a q-block of nt tiles in a row of ctx keys, q_len of them new (nt: one
+// range), and the first part of a q-block. A row is split by its own lengths, so that a row without cached
+// tokens is finished in one range whatever batch or table it comes with.
+__device__ __forceinline__ int split_range(const AttnArgs& a, int nt, int ctx, int q_len) {
+    if ((ctx + BN - 1) / BN < a.split_from || ctx / 4 < q_len) return nt;
+    return nt <= 4 * a.n_split ? min(nt, 4) : (nt + a.n_split - 1) / a.n_split;
 }
 __device__ __forceinline__ long part_index(const AttnArgs& a, int seq, int qb, int kvh) {
     return (((long)seq * a.n_qblocks + qb) * a.kv_heads + kvh) * a.n_split;
@@ -105,8 +107,8 @@ __device__ __forceinline__ long part_index(const AttnArgs& a, int seq, int qb, i
 // weights applied to V sum to one.
 //
 // SPLIT: a batch of few rows leaves most CUs idle (five 30-token questions over one 2,700-token state:
-// 40 workgroups of 43 tiles, 55.7 us; split 17.4 + 6.1). Then a workgroup takes one q-block and one range of its key tiles,
-// and writes its unnormalised fp32 O rows with their max and sum; attn_combine adds the ranges of a
+// 40 workgroups of 43 tiles, 54.9 us; split 13 and 6 for attn_combine). Then a workgroup takes one q-block and
+// one range of its key tiles, and writes its unnormalised fp32 O rows with their max and sum; attn_combine adds the ranges of a
 // row in their order. A q-block with a single range is finished here as in the unsplit kernel. A range
 // may lie past a row's last visible key: its max stays -inf and its probabilities 0.
 template <typename T, int NH, bool SPLIT>
@@ -124,9 +126,12 @@ __global__ __launch_bounds__(256, NH == 1 ? 2 : 1) void paged_prefill_attn_16(At
     // grid (kv_heads, q-block pairs, sequences): linear workgroup ids run KV head fastest,
     // and consecutive ids go round-robin to the 8 XCDs, so all q-block pairs of one
     // (sequence, KV head) run together on one XCD and share its L2 copy of the K/V pages
+    // SPLIT: grid (kv_heads, sequences, n_split ranges of each q-block), range 0 of all sequences side by
+    // side: where the contexts are short and have one range (a wide table), they spread over the chip as
+    // in the unsplit launch (16 rows of 130 keys under 4,096: 12.3 us, 16.4 with the ranges side by side)
     const int kvh = blockIdx.x;
     const int z = SPLIT ? 0 : blockIdx.y;
-    const int seq = blockIdx.z;
+    const int seq = SPLIT ? blockIdx.y : blockIdx.z;
     const int q0 = a.cu_seqlens_q[seq];
     const int q_len = a.cu_seqlens_q[seq + 1] - q0;
     const int ctx = a.context_lens[seq];
@@ -140,7 +145,7 @@ __global__ __launch_bounds__(256, NH == 1 ? 2 : 1) void paged_prefill_attn_16(At
     // sequence runs nq + 1 key tiles; the longer block goes first
     const int nq = (q_len + P - 1) / P;
     // (SPLIT: q-blocks past n_qblocks, rows longer than max_q_len, have no part)
-    const int qb_a = SPLIT ? a.n_qblocks - 1 - (int)(blockIdx.y / a.n_split) : nq - 1 - z, qb_b = z;
+    const int qb_a = SPLIT ? a.n_qblocks - 1 - (int)(blockIdx.z / a.n_split) : nq - 1 - z, qb_b = z;
     if (SPLIT ? qb_a >= nq : 2 * z >= nq) return;
     const int n_blocks = SPLIT || qb_a == qb_b ? 1 : 2;
     const int off = ctx - q_len;  // absolute position of the first new query
@@ -148,8 +153,9 @@ __global__ __launch_bounds__(256, NH == 1 ? 2 : 1) void paged_prefill_attn_16(At
     const int pmask = (1 << a.page_shift) - 1;
     auto block_tiles = [&](int qb) { return (off + min(q_len, (qb + 1) * P) - 1) / BN + 1; };
     // SPLIT: tiles i0 .. nt_a - 1 of the block's
-    const int nt_all = block_tiles(qb_a), range = SPLIT ? split_range(a, nt_all) : nt_all;
-    const int i0 = SPLIT ? (int)(blockIdx.y % a.n_split) * range : 0;
+    const int nt_all = block_tiles(qb_a), range = SPLIT ? split_range(a, nt_all, ctx, q_len) : nt_all;
+    const bool split = SPLIT && range < nt_all;
+    const int i0 = SPLIT ? (int)(blockIdx.z % a.n_split) * range : 0;
     if (SPLIT && i0 >= nt_all) return;
     const int nt_a = SPLIT ? min(nt_all, i0 + range) : nt_all;
     const int n_sched = nt_a + (n_blocks == 2 ? block_tiles(qb_b) : 0);
@@ -255,6 +261,8 @@ __global__ __launch_bounds__(256, NH == 1 ? 2 : 1) void paged_prefill_attn_16(At
     for (int db = 0; db < 4 * NH; ++db) acc_o[db] = f32x16{};
     float m_use = -INFINITY, l_run = 0.0f;
     const float c = a.scale_log2;
+    // a range whose keys so far are all masked or -inf adds nothing; a whole row of them is NaN, as unsplit
+    const float none = SPLIT && split ? 0.0f : -INFINITY;
 
     // Epilogue of block qb: o = O / l (both lane halves hold partial row sums), rounded to T,
     // then the output gate o = round(o) * round(sigmoid(gate)) as the reference rounds both.
@@ -341,7 +349,7 @@ __global__ __launch_bounds__(256, NH == 1 ? 2 : 1) void paged_prefill_attn_16(At
     };
     // probabilities of one half as the P.V operand (rounded to T), and their row sums
     auto half_p = [&](const f32x16& sv, v8* pf) {
-        const float mc = SPLIT && m_use == -INFINITY ? 0.0f : m_use * c;
+        const float mc = SPLIT && m_use == -INFINITY ? none : m_use * c;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             v8 t;
@@ -438,10 +446,10 @@ __global__ __launch_bounds__(256, NH == 1 ? 2 : 1) void paged_prefill_attn_16(At
         for (int i = i0; i < mf; ++i) step(i, no_mask);
         for (int i = max(mf, i0); i < nt_a; ++i) step(i, with_mask);
     }
-    if (SPLIT && range < nt_all) {
+    if (SPLIT && split) {
         const float l_tot = l_run + __shfl_xor(l_run, 32);
         if (!q_valid) return;  // rows past the sequence have no part (short suffixes fill half a block)
-        const long w = part_index(a, seq, qb_a, kvh) + blockIdx.y % a.n_split;
+        const long w = part_index(a, seq, qb_a, kvh) + blockIdx.z % a.n_split;
         float* const op = a.part + (w * 128 + row) * HD + 4 * g;
 #pragma unroll
         for (int db = 0; db < 4 * NH; ++db)
@@ -474,7 +482,7 @@ __global__ __launch_bounds__(256) void attn_combine(AttnArgs a) {
     const int q0 = a.cu_seqlens_q[seq], q_len = a.cu_seqlens_q[seq + 1] - q0, ctx = a.context_lens[seq];
     const int P = a.pos_per_block;
     if (q0 < 0 || q_len < 0 || q0 + q_len > a.n_tokens || q_len > ctx || qb * P >= q_len) return;
-    const int nt = (ctx - q_len + min(q_len, (qb + 1) * P) - 1) / BN + 1, range = split_range(a, nt);
+    const int nt = (ctx - q_len + min(q_len, (qb + 1) * P) - 1) / BN + 1, range = split_range(a, nt, ctx, q_len);
     if (range >= nt) return;  // finished by the attention kernel
     const int ns = (nt + range - 1) / range;
     const long w0 = part_index(a, seq, qb, kvh);
@@ -725,7 +733,7 @@ static int launch_split(const hk::AttnArgs* a, int n_seqs, hipStream_t stream) {
     static const bool configured = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                                        (int)(NH * ATTN16_LDS)) == hipSuccess;
     if (!configured) return HK_ERR_DEVICE;
-    hipLaunchKernelGGL(kern, dim3(a->kv_heads, a->n_qblocks * a->n_split, n_seqs), dim3(256), NH * ATTN16_LDS, stream, *a);
+    hipLaunchKernelGGL(kern, dim3(a->kv_heads, n_seqs, a->n_qblocks * a->n_split), dim3(256), NH * ATTN16_LDS, stream, *a);
     hipLaunchKernelGGL((attn_combine<T, NH>), dim3(a->kv_heads, a->n_qblocks * (128 / (NH == 1 ? 8 : 4)), n_seqs), dim3(256), 0,
                        stream, *a);
     return hipGetLastError() == hipSuccess ? HK_OK : HK_ERR_DEVICE;

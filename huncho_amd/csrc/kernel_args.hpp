@@ -25,9 +25,9 @@ struct AttnArgs {
     int num_pages;
     int n_tokens;
     int* fault;
-    // key-split kernel: each q-block's tiles in at most n_split ranges of at least split_tiles; part holds
-    // the ranges' unnormalised fp32 O rows, part_ml their (row max, row sum) pairs
-    int n_split, split_tiles, n_qblocks;
+    // key-split kernel: the tiles of each q-block of a row of at least split_from tiles in at most n_split
+    // ranges; part holds the ranges' unnormalised fp32 O rows, part_ml their (row max, row sum) pairs
+    int n_split, split_from, n_qblocks;
     float* part;
     float* part_ml;
 };

@@ -97,6 +97,54 @@ def test_a_fresh_row_keeps_its_bits(ctx):
     assert torch.equal(a, o[:1100]) and torch.equal(a, o[-1100:])
 
 
+def rows_of_one_batch(ctx, q_lens, ctx_lens, picks, spares, seed=11):
+    """The outputs of each pick of the rows, as batches of their own under tables with spare columns."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    r = lambda *s: torch.randn(s, generator=g, device="cuda").to(torch.bfloat16)
+    need = [(c + 15) // 16 for c in ctx_lens]
+    kp, vp = r(sum(need), 8, 16, 128), r(sum(need), 8, 16, 128)
+    first = np.concatenate([[0], np.cumsum(need)])
+    qg = [r(L, 16, 256) for L in q_lens]
+    out = []
+    for pick, spare in zip(picks, spares):
+        bt = np.zeros((len(pick), max(need[s] for s in pick) + spare), np.int32)
+        for i, s in enumerate(pick):
+            bt[i, :need[s]] = np.arange(first[s], first[s] + need[s])
+        q = torch.cat([qg[s] for s in pick])
+        cu = torch.tensor(np.concatenate([[0], np.cumsum([q_lens[s] for s in pick])]), dtype=torch.int32, device="cuda")
+        lens = torch.tensor([ctx_lens[s] for s in pick], dtype=torch.int32, device="cuda")
+        o = paged_prefill_attention(ctx, q[:, :, :128], kp, vp, torch.from_numpy(bt).cuda(), cu, lens,
+                                    max(q_lens[s] for s in pick), gate=q[:, :, 128:])
+        out.append(dict(zip(pick, o.split([q_lens[s] for s in pick]))))
+    assert ctx.take_faults() == 0
+    return out
+
+
+@pytest.mark.parametrize("fresh", [65, 600, 1000])
+def test_a_fresh_row_keeps_its_bits_beside_suffixes(ctx, fresh):
+    """Whether a row is split goes by its own lengths: a row without cached tokens gives the same bits alone,
+    under a wide table, and beside a suffix that is split."""
+    alone, wide, both = rows_of_one_batch(ctx, [fresh, 30], [fresh, 2700], [[0], [0], [0, 1]], [0, 250, 0])
+    assert torch.equal(alone[0], wide[0])
+    assert torch.equal(alone[0], both[0])
+
+
+def test_a_suffix_does_not_depend_on_the_table(ctx):
+    """The ranges of a suffix follow its context: the table's width does not change its bits."""
+    q_lens, ctx_lens = [30, 20, 33], [2700, 1300, 1100]
+    narrow, wide = rows_of_one_batch(ctx, q_lens, ctx_lens, [[0, 1, 2]] * 2, [0, 700])
+    assert all(torch.equal(narrow[s], wide[s]) for s in range(3))
+
+
+def test_many_launches_in_a_row(ctx):
+    """The counts of finished ranges are zero again after each launch, whatever the batch before was."""
+    a = [run(ctx, *x, 16, 8, 128, 16, torch.bfloat16, True, 9) for x in (([30] * 5, [2700] * 5), ([1], [4097]), ([128], [2048]))]
+    for _ in range(3):
+        for x, (o, e) in zip((([30] * 5, [2700] * 5), ([1], [4097]), ([128], [2048])), a):
+            o2, _ = run(ctx, *x, 16, 8, 128, 16, torch.bfloat16, True, 9)
+            assert e < TOL[torch.bfloat16] and torch.equal(o, o2)
+
+
 def test_nan_and_infinite_scores(ctx):
     """A key whose scores are +inf or NaN makes its rows NaN, as softmax does, in whichever range it lies;
     keys past a row's position do not reach it."""
