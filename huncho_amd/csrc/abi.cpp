@@ -8,6 +8,8 @@
 #include <string.h>
 
 #include <algorithm>
+#include <map>
+#include <mutex>
 #include <string>
 #include <utility>
 #include <vector>
@@ -44,6 +46,58 @@ extern "C" int hk_device_count(int* out) {
 
 extern "C" const char* hk_version(void) { return "huncho_rocm 0.1 (gfx950)"; }
 
+// Blocks of split scratch. One per device is kept when its context is destroyed, for the next context, and freed
+// with the device's last context.
+namespace {
+struct SplitPool {
+    std::mutex lock;
+    struct Device {
+        int contexts = 0;
+        void* spare = nullptr;
+    };
+    std::map<int, Device> devices;
+};
+SplitPool& split_pool() {
+    static SplitPool* pool = new SplitPool();  // outlives contexts that are destroyed as the process ends
+    return *pool;
+}
+
+// A block on the current device, or null
+void* split_block_take(int device, int new_contexts) {
+    void* p;
+    {
+        std::lock_guard<std::mutex> guard(split_pool().lock);
+        SplitPool::Device& d = split_pool().devices[device];
+        d.contexts += new_contexts;
+        p = d.spare;
+        d.spare = nullptr;
+    }
+    if (!p && hipMalloc(&p, kSplitScratch) != hipSuccess) {
+        (void)hipGetLastError();
+        p = nullptr;
+    }
+    return p;
+}
+
+// Work on the blocks has ended; the context is gone.
+void split_blocks_give(int device, void* a, void* b) {
+    void* drop[3] = {a, b, nullptr};
+    {
+        std::lock_guard<std::mutex> guard(split_pool().lock);
+        SplitPool::Device& d = split_pool().devices[device];
+        if (--d.contexts == 0) {
+            drop[2] = d.spare;
+            d.spare = nullptr;
+        } else if (!d.spare) {
+            d.spare = a;
+            drop[0] = nullptr;
+        }
+    }
+    for (void* p : drop)
+        if (p) hipFree(p);
+}
+}  // namespace
+
 extern "C" int hk_ctx_create(int device_ordinal, hk_ctx** out) {
     if (!out) return HK_ERR_INVALID;
     *out = nullptr;
@@ -73,6 +127,7 @@ extern "C" int hk_ctx_create(int device_ordinal, hk_ctx** out) {
         delete ctx;
         return HK_ERR_DEVICE;
     }
+    ctx->split_scratch = split_block_take(device_ordinal, 1);
     // the no-allocation entry point's scratch address on this device (retried on its first call
     // if this fails)
     hk_noalloc_scratch_init(device_ordinal);
@@ -86,11 +141,10 @@ extern "C" int hk_ctx_destroy(hk_ctx* ctx) {
     hipStreamSynchronize(ctx->stream);
     hk_noalloc_scratch_release(ctx);
     hk_blas_release(ctx);
-    if (ctx->split_scratch) {
-        hipDeviceSynchronize();  // its users may be on streams that the context has left
-        hipFree(ctx->split_scratch);
-    }
-    if (ctx->split_moved) hipEventDestroy(ctx->split_moved);
+    // the scratch's last use may be on a stream that the context has left
+    if (ctx->split_used && (ctx->split_done || ctx->split_stream != ctx->stream)) hipDeviceSynchronize();
+    split_blocks_give(ctx->device, ctx->split_scratch, ctx->split_first);
+    if (ctx->split_done) hipEventDestroy(ctx->split_done);
     if (ctx->fault_dev) hipFree(ctx->fault_dev);
     if (ctx->own_stream) hipStreamDestroy(ctx->own_stream);
     delete ctx;
@@ -99,18 +153,7 @@ extern "C" int hk_ctx_destroy(hk_ctx* ctx) {
 
 extern "C" int hk_ctx_set_stream(hk_ctx* ctx, void* hip_stream) {
     if (!ctx) return HK_ERR_INVALID;
-    const hipStream_t next = (hipStream_t)hip_stream;  // NULL is HIP's null stream
-    if (next != ctx->stream && ctx->split_scratch_used) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        const bool ok = hipStreamIsCapturing(ctx->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone &&
-                        (ctx->split_moved || hipEventCreateWithFlags(&ctx->split_moved, hipEventDisableTiming) == hipSuccess) &&
-                        hipEventRecord(ctx->split_moved, ctx->stream) == hipSuccess;
-        (void)hipGetLastError();
-        ctx->split_wait = true;
-        ctx->split_wait_all = !ok;
-        ctx->split_scratch_used = false;
-    }
-    ctx->stream = next;
+    ctx->stream = (hipStream_t)hip_stream;  // NULL is HIP's null stream
     return HK_OK;
 }
 
@@ -118,44 +161,47 @@ size_t hk_gdn_split_bytes(int n_tokens, int n_seqs, int heads) {
     return (size_t)(n_tokens / 64 + n_seqs) * heads * hk::HK_GDN_SPLIT_SLOT;
 }
 
-bool hk_split_scratch_reserve(hk_ctx* ctx, size_t bytes) {
-    if (bytes <= ctx->split_scratch_bytes) return true;
-    if (bytes > kSplitScratchMax) return false;
-    size_t size = 32u << 20;
-    while (size < bytes) size <<= 1;
-    bytes = size;
-    if (ctx->split_scratch) {
-        hipDeviceSynchronize();
-        hipFree(ctx->split_scratch);
-        ctx->split_scratch = nullptr;
-        ctx->split_scratch_bytes = 0;
-        ctx->split_scratch_used = ctx->split_wait = ctx->split_wait_all = false;
-    }
-    if (hipMalloc(&ctx->split_scratch, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        ctx->split_scratch = nullptr;
-        return false;
-    }
-    ctx->split_scratch_bytes = bytes;
-    return true;
-}
-
-// The scratch for a call on the context's stream, after the users on other streams, or null: too small
-// (grown only if may_alloc) or the stream is being captured (a graph may be replayed on any stream).
-static void* split_scratch_for(hk_ctx* ctx, size_t bytes, bool may_alloc) {
-    if (bytes > (may_alloc ? kSplitScratchMax : ctx->split_scratch_bytes)) return nullptr;
+// The scratch for a call on the context's stream, after its last use on another one; null: the call needs more
+// than there is, or the stream is being captured (a graph may be replayed on any stream).
+// An event per use costs 3 to 4 us (attention of 1 x 30 / 1030: 12.6 and 15.6), and an event on the stream that is
+// left cannot be had later, when that stream may be gone. So a context that stays on one stream records none. From
+// its first use on a second stream on it records one per use, and it leaves the block of the uses before,
+// whose end nothing marks, alone until it is destroyed. (A stream that got the handle of a destroyed one
+// counts as the same: hipStreamDestroy returns when the stream's work is done, measured with 42 ms of it.)
+static void* split_scratch_for(hk_ctx* ctx, size_t bytes) {
+    if (!ctx->split_scratch || bytes > kSplitScratch) return nullptr;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
         (void)hipGetLastError();
         return nullptr;
     }
-    if (!hk_split_scratch_reserve(ctx, bytes)) return nullptr;
-    if (ctx->split_wait) {
-        if (ctx->split_wait_all || hipStreamWaitEvent(ctx->stream, ctx->split_moved, 0) != hipSuccess) hipDeviceSynchronize();
-        ctx->split_wait = ctx->split_wait_all = false;
+    if (ctx->split_used && ctx->split_stream != ctx->stream) {
+        if (ctx->split_done) {
+            if (hipStreamWaitEvent(ctx->stream, ctx->split_done, 0) != hipSuccess) {
+                (void)hipGetLastError();
+                return nullptr;
+            }
+        } else {
+            if (hipEventCreateWithFlags(&ctx->split_done, hipEventDisableTiming) != hipSuccess) {
+                (void)hipGetLastError();
+                ctx->split_done = nullptr;
+                return nullptr;
+            }
+            ctx->split_first = ctx->split_scratch;
+            ctx->split_scratch = split_block_take(ctx->device, 0);
+            if (!ctx->split_scratch) return nullptr;
+        }
     }
-    ctx->split_scratch_used = true;
     return ctx->split_scratch;
+}
+
+// After the last launch of a use
+static void split_scratch_done(hk_ctx* ctx) {
+    ctx->split_used = true;
+    ctx->split_stream = ctx->stream;
+    if (!ctx->split_done || hipEventRecord(ctx->split_done, ctx->stream) == hipSuccess) return;
+    (void)hipGetLastError();
+    hipStreamSynchronize(ctx->stream);
 }
 
 extern "C" void* hk_ctx_own_stream(hk_ctx* ctx) { return ctx ? (void*)ctx->own_stream : nullptr; }
@@ -507,14 +553,13 @@ static int attn_split_from(long blocks, long pairs, int n_qblocks, int pos_per_b
     }
     return 0;
 }
-size_t hk_attn_split_bytes(int head_dim) { return (size_t)kAttnParts * 128 * (head_dim + 2) * sizeof(float); }
+static_assert((size_t)kAttnParts * 128 * (256 + 2) * sizeof(float) <= kSplitScratch, "every key-split launch fits");
 
 int hk_paged_prefill_attention_impl(hk_ctx* ctx, int dtype, const void* q, long q_tok, long q_head, const void* k_pool,
                                     const void* v_pool, int num_pages, int page_size, const int32_t* bt, int bt_stride,
                                     const int32_t* cu, const int32_t* ctxl, int n_seqs, int n_tokens, int max_q_len,
                                     int q_heads, int kv_heads, int head_dim, float scale, const void* gate,
-                                    long gate_tok, long gate_head, void* o, long o_tok, long o_head, int max_ctx,
-                                    bool may_alloc) {
+                                    long gate_tok, long gate_head, void* o, long o_tok, long o_head, int max_ctx) {
     if (!ctx) return HK_ERR_INVALID;
     if (int rc = check_dtype(ctx, dtype)) return rc;
     if (head_dim < 1 || head_dim > 256)
@@ -573,13 +618,14 @@ int hk_paged_prefill_attention_impl(hk_ctx* ctx, int dtype, const void* q, long 
                                                                 pos_per_block, tiles, &n);
         const size_t bytes = (size_t)(rows * n_qblocks * n) * 128 * (head_dim + 2) * sizeof(float);
         if (from) {
-            if (void* scratch = split_scratch_for(ctx, bytes, may_alloc)) {
+            if (void* scratch = split_scratch_for(ctx, bytes)) {
                 a.n_split = n;
                 a.split_from = from;
                 a.n_qblocks = n_qblocks;
                 a.part = (float*)scratch;
                 a.part_ml = a.part + (size_t)(rows * n_qblocks * n) * 128 * head_dim;
                 const int rc = hk_launch_paged_prefill_attention_split(dtype, &a, head_dim, n_seqs, ctx->stream);
+                split_scratch_done(ctx);
                 return rc ? hk_fail(ctx, rc, "attention launch failed") : HK_OK;
             }
         }
@@ -596,7 +642,7 @@ extern "C" int hk_paged_prefill_attention(hk_ctx* ctx, int dtype, const void* q,
                                           void* o, long o_tok, long o_head) {
     return hk_paged_prefill_attention_impl(ctx, dtype, q, q_tok, q_head, k_pool, v_pool, num_pages, page_size, bt,
                                            bt_stride, cu, ctxl, n_seqs, n_tokens, max_q_len, q_heads, kv_heads, head_dim,
-                                           scale, gate, gate_tok, gate_head, o, o_tok, o_head, 0, true);
+                                           scale, gate, gate_tok, gate_head, o, o_tok, o_head, 0);
 }
 
 // Whether the fp32 delta rule takes its three-kernel form (delta_rule_split.hip): few chains (pairs of a
@@ -615,7 +661,7 @@ int hk_gated_delta_chunked_rows(hk_ctx* ctx, int dtype, const void* q, long q_to
                                 const void* v, long v_tok, const float* g, const float* beta, const int32_t* cu,
                                 int n_seqs, int n_tokens, int heads, int k_heads, int dk, int dv,
                                 const float* initial_state, float* final_state, void* o, long o_tok,
-                                const float* const* init_rows, float* const* final_rows, bool may_alloc) {
+                                const float* const* init_rows, float* const* final_rows) {
     if (!ctx) return HK_ERR_INVALID;
     if (int rc = check_dtype(ctx, dtype)) return rc;
     // 128 x 128 states on the chunked MFMA kernels, others (each width in 1..256, at most 32768
@@ -640,8 +686,9 @@ int hk_gated_delta_chunked_rows(hk_ctx* ctx, int dtype, const void* q, long q_to
                   final_state, o, o_tok, heads, n_tokens, ctx->fault_dev, init_rows, final_rows};
     // (the split form reads q and k after it has written part of o: o in their place stays with one kernel)
     if (mfma && dtype == HK_F32 && delta_split_takes(n_seqs, n_tokens, heads) && o != q && o != k) {
-        if (void* scratch = split_scratch_for(ctx, hk_delta_split_bytes(n_tokens, n_seqs, heads), may_alloc)) {
+        if (void* scratch = split_scratch_for(ctx, hk_delta_split_bytes(n_tokens, n_seqs, heads))) {
             const int rc = hk_launch_delta_split(&a, n_seqs, n_tokens / 64 + n_seqs, scratch, ctx->stream);
+            split_scratch_done(ctx);
             return rc ? hk_fail(ctx, rc, "gated delta launch failed") : HK_OK;
         }
     }
@@ -655,7 +702,7 @@ extern "C" int hk_gated_delta_chunked(hk_ctx* ctx, int dtype, const void* q, lon
                                       int n_seqs, int n_tokens, int heads, int k_heads, int dk, int dv,
                                       const float* initial_state, float* final_state, void* o, long o_tok) {
     return hk_gated_delta_chunked_rows(ctx, dtype, q, q_tok, k, k_tok, v, v_tok, g, beta, cu, n_seqs, n_tokens, heads,
-                                       k_heads, dk, dv, initial_state, final_state, o, o_tok, nullptr, nullptr, true);
+                                       k_heads, dk, dv, initial_state, final_state, o, o_tok, nullptr, nullptr);
 }
 
 int hk_gdn_prep_rows(hk_ctx* ctx, int dtype, const void* mixed, long mixed_tok, const float* conv_w, int conv_k,
@@ -743,7 +790,7 @@ int hk_gdn_fused_rows(hk_ctx* ctx, int dtype, const void* mixed, long mixed_tok,
                       float eps, const int32_t* cu, int n_seqs, int n_tokens, int heads, int k_heads,
                       const float* initial_state, float* final_state, void* out, long out_tok,
                       const float* const* init_rows, float* const* final_rows, const void* const* hist_rows,
-                      void* const* tail_rows, bool may_alloc) {
+                      void* const* tail_rows) {
     if (!ctx) return HK_ERR_INVALID;
     if (dtype != HK_BF16 && dtype != HK_F16)
         return hk_fail(ctx, HK_ERR_UNSUPPORTED, "fused Gated DeltaNet layer: 16-bit dtypes only (got %d)", dtype);
@@ -771,8 +818,9 @@ int hk_gdn_fused_rows(hk_ctx* ctx, int dtype, const void* mixed, long mixed_tok,
     hk::GdnFusedArgs fa{mixed, mixed_tok, conv_w, (int)conv_dim, conv_hist, conv_tail_out, ba, ba_tok, b_col, a_col,
                         base_g, dt_bias, 1.0f / sqrtf(128.0f), k_heads, z, z_tok, norm_w, eps, hist_rows, tail_rows};
     if (gdn_split_takes(n_seqs, n_tokens, heads)) {
-        if (void* scratch = split_scratch_for(ctx, hk_gdn_split_bytes(n_tokens, n_seqs, heads), may_alloc)) {
+        if (void* scratch = split_scratch_for(ctx, hk_gdn_split_bytes(n_tokens, n_seqs, heads))) {
             const int rc = hk_launch_gdn16_split(dtype, &a, &fa, n_seqs, n_tokens / 64 + n_seqs, scratch, ctx->stream);
+            split_scratch_done(ctx);
             return rc ? hk_fail(ctx, rc, "fused Gated DeltaNet launch failed") : HK_OK;
         }
     }
@@ -787,7 +835,7 @@ extern "C" int hk_gdn_fused(hk_ctx* ctx, int dtype, const void* mixed, long mixe
                             int k_heads, const float* initial_state, float* final_state, void* out, long out_tok) {
     return hk_gdn_fused_rows(ctx, dtype, mixed, mixed_tok, conv_w, conv_k, conv_hist, conv_tail_out, ba, ba_tok, b_col,
                              a_col, base_g, dt_bias, z, z_tok, norm_w, eps, cu, n_seqs, n_tokens, heads, k_heads,
-                             initial_state, final_state, out, out_tok, nullptr, nullptr, nullptr, nullptr, true);
+                             initial_state, final_state, out, out_tok, nullptr, nullptr, nullptr, nullptr);
 }
 
 // ---------------------------------------------------------------------------

@@ -20,20 +20,19 @@ struct hk_ctx {
     int* fault_dev = nullptr;
     std::string last_error;
     hk_blas* blas = nullptr;
-    // Scratch of the kernels that split few, long rows over the chip (gdn16_split.hip, the key-split
-    // attention): at most kSplitScratchMax bytes, kept until the context is destroyed. Work on it is ordered by the stream; when the context moves to
-    // another stream, split_moved marks the end of the old stream's use and the next use waits for it.
+    // Scratch of the kernels that split few, long rows over the chip (gdn16_split.hip, delta_rule_split.hip, the
+    // key-split attention): kSplitScratch bytes from hk_ctx_create on (null if they could not be had), so that
+    // which kernel a call takes follows from its sizes. Work on it is ordered by the stream (split_stream: of
+    // the last use). split_done, from the context's first use on a second stream on: the end of the last use;
+    // split_first: the block of the uses before that.
     void* split_scratch = nullptr;
-    size_t split_scratch_bytes = 0;
-    bool split_scratch_used = false;     // on the current stream, since the last move
-    hipEvent_t split_moved = nullptr;
-    bool split_wait = false, split_wait_all = false;
+    void* split_first = nullptr;
+    hipStream_t split_stream = nullptr;
+    hipEvent_t split_done = nullptr;
+    bool split_used = false;
 };
 constexpr int kAttnParts = 512;  // most parts of a key-split attention launch, of at most half as many q-blocks
-constexpr size_t kSplitScratchMax = 512u << 20;
-// Ensures `bytes` of scratch (rounded up to a power of two, at least 32 MiB); frees and reallocates a smaller one after waiting
-// for its users. false if bytes exceed the limit or the allocation fails.
-bool hk_split_scratch_reserve(hk_ctx* ctx, size_t bytes);
+constexpr size_t kSplitScratch = 512u << 20;
 // Bytes for the chunks of n_tokens tokens in n_seqs rows.
 size_t hk_gdn_split_bytes(int n_tokens, int n_seqs, int heads);
 size_t hk_delta_split_bytes(int n_tokens, int n_seqs, int heads);
@@ -56,16 +55,12 @@ int hk_gemm_xwt(hk_ctx* ctx, int dtype, int n, int out, int in, const void* x, l
 int hk_gemm_xwt_cd(hk_ctx* ctx, int dtype, int cd_dtype, int n, int out, int in, const void* x, long ldx,
                    const void* w, long ldw, void* y, long ldy, const void* c, long ldc, float alpha, float beta);
 
-// hk_paged_prefill_attention with a bound on the batch's context lengths (0: what the block tables can
-// hold) and the choice whether the split scratch may be allocated or grown (not inside a forward).
+// hk_paged_prefill_attention with a bound on the batch's context lengths (0: what the block tables can hold).
 int hk_paged_prefill_attention_impl(hk_ctx* ctx, int dtype, const void* q, long q_tok, long q_head, const void* k_pool,
                                     const void* v_pool, int num_pages, int page_size, const int32_t* bt, int bt_stride,
                                     const int32_t* cu, const int32_t* ctxl, int n_seqs, int n_tokens, int max_q_len,
                                     int q_heads, int kv_heads, int head_dim, float scale, const void* gate,
-                                    long gate_tok, long gate_head, void* o, long o_tok, long o_head, int max_ctx,
-                                    bool may_alloc);
-// Most scratch bytes that one key-split attention launch takes.
-size_t hk_attn_split_bytes(int head_dim);
+                                    long gate_tok, long gate_head, void* o, long o_tok, long o_head, int max_ctx);
 
 // Two projections of the same x rows, Y = X W^T and Y2 = X W2^T (contiguous weights and outputs).
 int hk_gemm_xwt_pair(hk_ctx* ctx, int dtype, int n, int in, const void* x, long ldx, int out, const void* w, void* y,

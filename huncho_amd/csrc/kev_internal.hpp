@@ -73,7 +73,7 @@ int hk_gated_delta_chunked_rows(hk_ctx* ctx, int dtype, const void* q, long q_to
                                 const void* v, long v_tok, const float* g, const float* beta, const int32_t* cu,
                                 int n_seqs, int n_tokens, int heads, int k_heads, int dk, int dv,
                                 const float* initial_state, float* final_state, void* o, long o_tok,
-                                const float* const* init_rows, float* const* final_rows, bool may_alloc);
+                                const float* const* init_rows, float* const* final_rows);
 int hk_gdn_prep_rows(hk_ctx* ctx, int dtype, const void* mixed, long mixed_tok, const float* conv_w, int conv_k,
                      const void* conv_hist, const void* ba, long ba_tok, int b_col, int a_col, const float* base_g,
                      const float* dt_bias, const int32_t* cu, int n_seqs, int n_tokens, int heads, int k_heads,
@@ -85,4 +85,4 @@ int hk_gdn_fused_rows(hk_ctx* ctx, int dtype, const void* mixed, long mixed_tok,
                       float eps, const int32_t* cu, int n_seqs, int n_tokens, int heads, int k_heads,
                       const float* initial_state, float* final_state, void* out, long out_tok,
                       const float* const* init_rows, float* const* final_rows, const void* const* hist_rows,
-                      void* const* tail_rows, bool may_alloc);
+                      void* const* tail_rows);

@@ -229,16 +229,6 @@ extern "C" int hk_kev_model_create(hk_ctx* ctx, int dtype, const hk_kev_config* 
         hk_rope_fill_table(c.rotary_dim, c.rope_theta, c.max_context, dtype, cs.data(), sn.data());
         if ((rc = upload_f32(m, cs, &m->rope_cos)) || (rc = upload_f32(m, sn, &m->rope_sin))) return fail(rc);
     }
-    // scratch for the key-split attention, and for up to four rows of max_context tokens through the Gated
-    // DeltaNet layers, at most half of the limit, so that no forward allocates (batches that do not fit
-    // run the layer without it)
-    if (dtype != HK_F32 && (c.head_dim == 128 || c.head_dim == 256)) hk_split_scratch_reserve(ctx, hk_attn_split_bytes(c.head_dim));
-    if ((dtype == HK_F32 || c.conv_k == 4) && c.lin_key_dim == 128 && c.lin_v_dim == 128) {
-        const int tokens = 4 * (c.max_context < 65536 ? c.max_context : 65536);
-        const size_t want = dtype == HK_F32 ? hk_delta_split_bytes(tokens, 4, c.lin_n_v_heads)
-                                            : hk_gdn_split_bytes(tokens, 4, c.lin_n_v_heads);
-        hk_split_scratch_reserve(ctx, want < kSplitScratchMax / 2 ? want : kSplitScratchMax / 2);
-    }
     hipStreamSynchronize(nullptr);  // the weight copies, on the null stream, are complete before the
                                     // context's stream (non-blocking) uses them
     *out = m;
@@ -482,8 +472,7 @@ int kev_forward_impl(hk_kev_model* m, const int32_t* ids, const int32_t* cu_dev,
                                       a_col, L.base_g, L.dt_bias, (char*)b.big + (size_t)m->conv_dim * e, rows, L.norm_w,
                                       c.eps, cu_dev, n_seqs, n, Hv, Hk, nullptr, nullptr, b.o, (long)Hv * dv,
                                       view ? view->init_rows[gi] : nullptr, view ? view->final_rows[gi] : nullptr,
-                                      view ? view->hist_rows[gi] : nullptr, view ? view->tail_rows[gi] : nullptr,
-                                      false));
+                                      view ? view->hist_rows[gi] : nullptr, view ? view->tail_rows[gi] : nullptr));
             } else {
                 // the cache's per-sequence conv tails and states, as in the fused path
                 RUN(hk_gdn_prep_rows(ctx, dt, b.big, rows, L.conv_w, c.conv_k, nullptr, b.ba, m->ba_rows, b_col, a_col,
@@ -493,7 +482,7 @@ int kev_forward_impl(hk_kev_model* m, const int32_t* ids, const int32_t* cu_dev,
                 RUN(hk_gated_delta_chunked_rows(ctx, dt, b.q, (long)Hk * dk, b.k, (long)Hk * dk, b.v, (long)Hv * dv,
                                                 b.g, b.beta, cu_dev, n_seqs, n, Hv, Hk, dk, dv, nullptr, nullptr, b.o,
                                                 (long)Hv * dv, view ? view->init_rows[gi] : nullptr,
-                                                view ? view->final_rows[gi] : nullptr, false));
+                                                view ? view->final_rows[gi] : nullptr));
                 RUN(hk_gated_rms_norm(ctx, dt, b.o, (char*)b.big + (size_t)m->conv_dim * e, rows, Hv, L.norm_w, c.eps,
                                       n * Hv, dv, b.o));
             }
@@ -516,7 +505,7 @@ int kev_forward_impl(hk_kev_model* m, const int32_t* ids, const int32_t* cu_dev,
             RUN(hk_paged_prefill_attention_impl(ctx, dt, qg, rows, 2 * hd, k_pool, v_pool, num_pages, c.page_size, bt,
                                                 bt_stride, cu_dev, ctx_lens, n_seqs, n, max_len, Hq, Hkv, hd,
                                                 (float)(1.0 / sqrt((double)hd)), qg + (size_t)hd * e, rows, 2 * hd, b.o,
-                                                (long)Hq * hd, hd, view ? view->max_ctx : max_len, false));
+                                                (long)Hq * hd, hd, view ? view->max_ctx : max_len));
             RUN(hk_gemm_xwt_cd(ctx, dt, xdt, n, H, Hq * hd, b.o, Hq * hd, L.w_o, Hq * hd, b.x, H, b.x, H, 1.0f, 1.0f));
         }
         RUN(norm_x(m, b.x, L.post_norm, n, b.h));

@@ -71,14 +71,17 @@ typedef struct {
 } hk_device_info_t;
 
 /* ---- context (replaces device selection, crates/huncho-backend/src/device.rs:12-72) ---- */
-/* Fails with HK_ERR_UNSUPPORTED when no GPU is visible (hipGetDeviceCount == 0). */
+/* Fails with HK_ERR_UNSUPPORTED when no GPU is visible (hipGetDeviceCount == 0).
+ * The context holds 512 MiB of device scratch for batches of few, long rows (hk_gdn_fused,
+ * hk_gated_delta_chunked in fp32, hk_paged_prefill_attention on suffixes, and the models' layers), from
+ * here to hk_ctx_destroy (another 512 MiB once it has used it on two streams). Which kernel a call takes follows from its sizes,
+ * and whether its stream is being captured: a captured call runs without the scratch, as does a context
+ * that could not have it. For the fp32 delta rule and the suffix attention the two differ by the
+ * rounding of their sums. */
 int hk_ctx_create(int device_ordinal, hk_ctx** out);
 int hk_ctx_destroy(hk_ctx* ctx);
 /* Work is ordered on this hipStream_t from now on (NULL: HIP's null stream). A new
- * context uses its own default-priority stream, returned by hk_ctx_own_stream. The scratch that
- * the context keeps for batches of few, long rows (at most 512 MiB, grown by per-op calls and at
- * model creation, freed with the context) follows it: the first use on the new stream waits for
- * the old stream's last. The stream that the context leaves must still exist at this call. */
+ * context uses its own default-priority stream, returned by hk_ctx_own_stream. */
 int hk_ctx_set_stream(hk_ctx* ctx, void* hip_stream);
 void* hk_ctx_stream(hk_ctx* ctx);
 void* hk_ctx_own_stream(hk_ctx* ctx);
