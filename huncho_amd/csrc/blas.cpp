@@ -216,36 +216,49 @@ static bool few_rows_takes(int dtype, int epi, const hk::GemmArgs& a) {
     return (((uintptr_t)a.x | (uintptr_t)a.w | (uintptr_t)a.c | (uintptr_t)a.y | (uintptr_t)a.w2 | (uintptr_t)a.y2) & 15) == 0;
 }
 
-// A model's projection takes the few-row kernel where its estimated time (us) is no more than about the
-// library's. Kernel times beside the library's choice, bf16: 8192 x 1024 at 169 rows 9.5 against 13.6, at
-// 450 rows 15.5 against 16.5, at 600 rows 22.9 against 17.3 (library); 6144 x 1024 at 600 rows 15.6 against
-// 19.2; 1024 x 3584 + residual at 300 rows 13.5 against 14.7, at 1700 rows 25.5 against 29, at 2704 rows
-// 38.7 against 36 (library); 2304 x 768 at 1200 rows 10.0 against 17.1. Both give the same bits.
-static bool few_rows_wins(int epi, const hk::GemmArgs& a) {
-    const float k = (float)a.K / 1024.0f;
-    const float lib = 5.0f + 2.2f * k + 0.9f * 2e-9f * (float)a.M * (float)(a.N + a.N2) * (float)a.K;
-    return 2.2f + k * hk_gemm_few_rows_cost(epi, &a) <= 1.1f * lib;
+// Estimated times (us) of a product on the few-row kernel and on the library's.
+static float few_rows_us(int epi, const hk::GemmArgs& a) {
+    return 2.2f + (float)a.K / 1024.0f * hk_gemm_few_rows_cost(epi, &a);
+}
+static float library_us(const hk::GemmArgs& a) {
+    return 5.0f + 2.2f * (float)a.K / 1024.0f + 0.9f * 2e-9f * (float)a.M * (float)a.N * (float)a.K;
+}
+// A model's projection takes the few-row kernel where its estimate is the lower one by 7 %. Measured beside the
+// library's choice (bf16, weights from HBM): 8192 x 1024 at 169 rows 9.3 against 12.7, at 360 rows 14.3 and
+// 13.8, at 512 rows 17.0 and 14.8, at 600 (library) 22 and 16.4; 1024 x 3584 + residual at 300 rows 12.3 against
+// 17.2, at 1024 (library) 19.6 and 18.9, at 4096 (library) 46.1 and 36.6; 768 x 1152 + residual at 1700 rows 9.8 against
+// 10.6, at 2704 (library) 14.6 and 12.7; 32 x 1024 at 16384 rows 5.4 against 10.1, at 32768 (library) 11.7 and 13.2.
+// The few-row kernel's sums do not depend on the number of rows. The library's choice for some small batches
+// adds in another order, and there the two differ by the rounding of their sums.
+static bool few_rows_wins(int epi, const hk::GemmArgs& a) { return few_rows_us(epi, a) <= 0.93f * library_us(a); }
+// The way such a projection takes, estimated
+static float projection_us(const hk::GemmArgs& a) {
+    return std::min(few_rows_us(hk::EPI_STORE, a), 0.93f * library_us(a));
 }
 
 int hk_gemm_xwt_pair(hk_ctx* ctx, int dtype, int n, int in, const void* x, long ldx, int out, const void* w, void* y,
                      int out2, const void* w2, void* y2) {
     const hk::GemmArgs a{x, w, nullptr, y, ldx, in, 0, out, n, out, in, w2, y2, out2, out2};
+    const hk::GemmArgs a1{x, w, nullptr, y, ldx, in, 0, out, n, out, in, nullptr, nullptr, 0, 0},
+        a2{x, w2, nullptr, y2, ldx, in, 0, out2, n, out2, in, nullptr, nullptr, 0, 0};
+    // (one launch for both: 8192 and 32 columns x 1024 at 169 rows 10.7 us, two of this kernel 13.9; at 360 rows
+    // 15.6 and 18.9; at 200 rows the columns of the second are a round of tiles of their own, 14.5 both ways)
     if (n > 0 && ctx->blas && !ctx->blas->autotune && few_rows_takes(dtype, hk::EPI_STORE, a) &&
-        few_rows_wins(hk::EPI_STORE, a))
+        few_rows_us(hk::EPI_STORE, a) <= projection_us(a1) + projection_us(a2))
         return hk_launch_gemm_few_rows(dtype, hk::EPI_STORE, &a, ctx->stream) ? hk_fail(ctx, HK_ERR_DEVICE, "gemm launch failed")
                                                                            : HK_OK;
     if (int rc = hk_gemm_xwt(ctx, dtype, n, out, in, x, ldx, w, in, y, out, nullptr, 0, 1.0f, 0.0f)) return rc;
     return hk_gemm_xwt(ctx, dtype, n, out2, in, x, ldx, w2, in, y2, out2, nullptr, 0, 1.0f, 0.0f);
 }
 
-// The encoder's GeGLU in the projection's epilogue, wherever the few-row kernel would take the projection: one
-// launch and one pass over 2 inter columns less (encoder of 22 layers, 653 rows: 1256 -> 1234 us; two runs
-// of one side differ by 0.2 %). In the library's range the pass on its own is the faster one (erf in the epilogue
-// of large tiles leaves the matrix cores idle).
+// The encoder's GeGLU in the projection's epilogue, one launch and one pass over 2 inter columns less (encoder of
+// 22 layers, 653 rows: 1256 -> 1234 us; two runs of one side differ by 0.2 %): where the estimate is below that
+// of the projection and a pass of 2.5 us. For many rows the pass on its own is the faster way (erf in
+// the epilogue of large tiles leaves the matrix cores idle).
 bool hk_gemm_geglu_few_rows(hk_ctx* ctx, int dtype, int n, int inter, int in, const void* x, const void* w, void* y, int* rc) {
     const hk::GemmArgs a{x, w, nullptr, y, in, in, 0, inter, n, 2 * inter, in, nullptr, nullptr, 0, 0};
     if (n <= 0 || !ctx->blas || ctx->blas->autotune || 4L * inter * in >= 1L << 31 || !few_rows_takes(dtype, hk::EPI_GEGLU, a) ||
-        !few_rows_wins(hk::EPI_GEGLU, a))
+        few_rows_us(hk::EPI_GEGLU, a) > projection_us(a) + 2.5f)
         return false;
     *rc = hk_launch_gemm_few_rows(dtype, hk::EPI_GEGLU, &a, ctx->stream) ? hk_fail(ctx, HK_ERR_DEVICE, "gemm launch failed")
                                                                          : HK_OK;
@@ -409,7 +422,8 @@ int hk_gemm_native(hk_ctx* ctx, int dtype, int epi, int n, int out, int in, cons
     hk::GemmArgs a{x, w, epi == hk::EPI_RESIDUAL ? c : nullptr, y, ldx, ldw, ldc, ldy, n, out, in, nullptr, nullptr, 0, 0};
     // The 256 x 256 tiles of gemm.hip cost about 30 K / 1024 us per round of 256 workgroups, however few
     // the rows; the few-row kernel's tiles less while there are few of them (7168 x 1024 SwiGLU at 600
-    // rows 21 against 34 us, at 1700 rows 39 against 35; 1024 x 3584 at 2704 rows 38.7 against 99).
+    // rows 21 against 33 us, at 1700 rows 39 and 37; 1024 x 3584 + residual at 4096 rows 46 against 99, at 8192 rows
+    // 88 against 109, at 16384 rows 165 and 115).
     const int tiles = out / 256 * ((n + 255) / 256);
     if (few_rows_takes(dtype, epi, a) && hk_gemm_few_rows_cost(epi, &a) < 30.0f * (float)((tiles + 255) / 256))
         return hk_launch_gemm_few_rows(dtype, epi, &a, ctx->stream) ? hk_fail(ctx, HK_ERR_DEVICE, "gemm launch failed") : HK_OK;

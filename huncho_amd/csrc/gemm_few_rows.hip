@@ -222,31 +222,39 @@ __global__ __launch_bounds__(NTHREADS, 2) void gemm_few_rows(GemmArgs a) {
 }  // namespace gemm_few
 }  // namespace hk
 
-// The tiles and their cost in units of K / 1024 us, fitted to the times of 8 to 2704 rows of the
-// projections above: flat while the tiles fit the chip at once; for more, rising with their number
-// (slope), or in rounds of 512 (two workgroups per CU) for the tiles whose second workgroup on a CU
-// takes as long as the first.
+// The tiles and their cost in units of K / 1024 us (beside about 2.2 us of launch and first loads), fitted to the
+// times of every tile over ten projections of the models (32 to 8192 columns, K 768 to 3584) at 34 to 32768 rows:
+// flat while the tiles fit the chip at once; for more, rising with their number (slope), with a step where the
+// third workgroup of a CU begins (past_512), or in rounds of 512 (two workgroups per CU) for the tiles whose
+// second workgroup on a CU takes as long as the first. X rows that do not stay in an XCD's L2 are read
+// once more for every column tile, at 17 TB/s over the chip: 1024 x 3584 at 4096 rows takes 66.8 us in
+// 64-column tiles and 46.1 in 128-column ones, of the same number and size.
 namespace {
 struct Tile {
     int nb, mb;
-    float first, slope, round;
+    float first, slope, past_512, round;
 };
-constexpr Tile kTiles[] = {{1, 1, 2.5f, 0.0092f, 0.0f}, {1, 2, 3.1f, 0.0125f, 0.0f}, {2, 2, 5.2f, 0.0145f, 0.0f},
-                           {2, 3, 5.3f, 0.0f, 9.5f},    {2, 4, 6.2f, 0.0f, 10.8f},   {4, 2, 6.3f, 0.0f, 11.2f}};
+constexpr Tile kTiles[] = {{1, 1, 2.5f, 0.0094f, 0.0f, 0.0f}, {1, 2, 2.9f, 0.0135f, 0.0f, 0.0f}, {2, 2, 5.1f, 0.0153f, 4.2f, 0.0f},
+                           {2, 3, 5.3f, 0.0f, 0.0f, 8.2f},    {2, 4, 6.2f, 0.0f, 0.0f, 10.8f},   {4, 2, 6.9f, 0.0f, 0.0f, 10.9f}};
 constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 
-long n_tiles(const hk::GemmArgs* a, const Tile& t) {
+long col_tiles(const hk::GemmArgs* a, const Tile& t) {
     const int w = 32 * t.nb;
-    return (long)((a->N + w - 1) / w + (a->N2 + w - 1) / w) * ((a->M + 32 * t.mb - 1) / (32 * t.mb));
+    return (a->N + w - 1) / w + (a->N2 + w - 1) / w;
 }
+long n_tiles(const hk::GemmArgs* a, const Tile& t) { return col_tiles(a, t) * ((a->M + 32 * t.mb - 1) / (32 * t.mb)); }
 
 int best_tile(int epi, const hk::GemmArgs* a, float* cost) {
+    const bool x_in_l2 = 2.0f * (float)a->M * (float)a->K < 5e6f;
     int best = -1;
     for (int i = 0; i < kNumTiles; ++i) {
         if ((epi == hk::EPI_SWIGLU || epi == hk::EPI_GEGLU) && (kTiles[i].nb % 2 || kTiles[i].mb % 2)) continue;  // four waves' 32 x 32 blocks
         const Tile& k = kTiles[i];
         const long n = n_tiles(a, k);
-        const float c = n <= 256 ? k.first : k.round > 0.0f ? k.round * (float)((n + 511) / 512) : k.first + k.slope * (float)(n - 256);
+        float c = n <= 256 ? k.first
+                  : k.round > 0.0f ? k.round * (float)((n + 511) / 512)
+                                   : k.first + k.slope * (float)(n - 256) + (n > 512 ? k.past_512 : 0.0f);
+        if (!x_in_l2) c += (float)(col_tiles(a, k) * a->M) * (2048.0f / 17e6f);
         if (best < 0 || c < *cost) {
             best = i;
             *cost = c;
@@ -303,7 +311,7 @@ static int launch_type(int epi, const hk::GemmArgs* a, hipStream_t stream) {
     }
 }
 
-// Cost of the best tile in units of K / 1024 us (beside about 2 us of launch and first loads).
+// Cost of the best tile in units of K / 1024 us (beside about 2.2 us of launch and first loads).
 extern "C" float hk_gemm_few_rows_cost(int epi, const hk::GemmArgs* a) {
     float cost = 0.0f;
     best_tile(epi, a, &cost);
