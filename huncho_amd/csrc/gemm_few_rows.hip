@@ -4,13 +4,14 @@
 //
 // What bounds such a product is the latency of streaming the weight rows once through too few
 // workgroups, not MFMA. So the tile is small, 32 NB columns x 32 MB rows shared by four waves (2 x 2),
-// K runs in steps of 64 through a ring of ST stages in LDS, which keeps up to 140 KB of loads in flight
-// per CU; where there are tiles enough two workgroups share a CU, and one's loads cover the other's
+// K runs in steps of 64 through a ring of ST stages in LDS, of which ST - U are being loaded (80 to 120 KB per
+// CU); where there are tiles enough two workgroups share a CU, and one's loads cover the other's
 // reads, barrier and epilogue.
 // Each output is one chain of fp32 accumulations over K in order, whatever the tile or the number of
 // rows, so a row's result does not change with the batch it comes in: SwiGLU on the 32x32x16 products
 // of gemm.hip (the same bits as that kernel), store and residual on 16x16x32 products (the same bits as
-// the library's kernels of these projections, so prefixes computed alone and whole rows agree as before).
+// the library's kernels of the large batches, so a prefix computed alone agrees with whole rows in a batch; for some
+// small batches the library's choice adds in another order, which the sums here replaced).
 // (A split of K over the four waves, each with a ring of its own, ran as fast but gave other sums.)
 //
 // Measured (us, bf16, weights rotated through 600 MB so that they come from HBM; gemm.hip beside it):
@@ -284,30 +285,26 @@ static int launch_one(const hk::GemmArgs* a, hipStream_t stream) {
 }
 
 template <typename T, int EPI>
-static int launch_epi(const hk::GemmArgs* a, hipStream_t stream) {
-    // Tiles that fit the chip at once run one workgroup per CU with a ring of 140 KB, more tiles two with
-    // half of it.
-    float cost;
-    const int i = best_tile(EPI, a, &cost);
-    const bool deep = n_tiles(a, kTiles[i]) <= 256;
+static int launch_epi(const hk::GemmArgs* a, int i, int deep, hipStream_t stream) {
     switch (i) {
         case 0: return deep ? launch_one<T, EPI, 0, 18, 4>(a, stream) : launch_one<T, EPI, 0, 9, 4>(a, stream);
         case 1: return deep ? launch_one<T, EPI, 1, 12, 4>(a, stream) : launch_one<T, EPI, 1, 6, 2>(a, stream);
         case 2: return deep ? launch_one<T, EPI, 2, 9, 4>(a, stream) : launch_one<T, EPI, 2, 5, 2>(a, stream);
         case 3: return deep ? launch_one<T, EPI, 3, 8, 2>(a, stream) : launch_one<T, EPI, 3, 4, 1>(a, stream);
         case 4: return deep ? launch_one<T, EPI, 4, 6, 2>(a, stream) : launch_one<T, EPI, 4, 3, 1>(a, stream);
-        default: return deep ? launch_one<T, EPI, 5, 6, 2>(a, stream) : launch_one<T, EPI, 5, 3, 1>(a, stream);
+        case 5: return deep ? launch_one<T, EPI, 5, 6, 2>(a, stream) : launch_one<T, EPI, 5, 3, 1>(a, stream);
+        default: return HK_ERR_DEVICE;
     }
 }
 
 template <typename T>
-static int launch_type(int epi, const hk::GemmArgs* a, hipStream_t stream) {
+static int launch_type(int epi, const hk::GemmArgs* a, int i, int deep, hipStream_t stream) {
     switch (epi) {
-        case hk::EPI_RESIDUAL: return launch_epi<T, hk::EPI_RESIDUAL>(a, stream);
-        case hk::EPI_RESIDUAL_F32: return launch_epi<T, hk::EPI_RESIDUAL_F32>(a, stream);
-        case hk::EPI_SWIGLU: return launch_epi<T, hk::EPI_SWIGLU>(a, stream);
-        case hk::EPI_GEGLU: return launch_epi<T, hk::EPI_GEGLU>(a, stream);
-        default: return launch_epi<T, hk::EPI_STORE>(a, stream);
+        case hk::EPI_RESIDUAL: return launch_epi<T, hk::EPI_RESIDUAL>(a, i, deep, stream);
+        case hk::EPI_RESIDUAL_F32: return launch_epi<T, hk::EPI_RESIDUAL_F32>(a, i, deep, stream);
+        case hk::EPI_SWIGLU: return launch_epi<T, hk::EPI_SWIGLU>(a, i, deep, stream);
+        case hk::EPI_GEGLU: return launch_epi<T, hk::EPI_GEGLU>(a, i, deep, stream);
+        default: return launch_epi<T, hk::EPI_STORE>(a, i, deep, stream);
     }
 }
 
@@ -321,6 +318,16 @@ extern "C" float hk_gemm_few_rows_cost(int epi, const hk::GemmArgs* a) {
 // dtype16: 1 = bf16, 2 = fp16. The caller has checked: N and N2 % 8 == 0 (SwiGLU, GeGLU: N % 32), K % 64 == 0,
 // 16-byte aligned rows (ld % 8 == 0) and row strides below 2^22 elements (32-bit copy offsets).
 extern "C" int hk_launch_gemm_few_rows(int dtype16, int epi, const hk::GemmArgs* a, hipStream_t stream) {
+    float cost;
+    const int i = best_tile(epi, a, &cost);
+    // Tiles that fit the chip at once run one workgroup per CU with a ring of up to 160 KB, more tiles two with
+    // half of it.
+    return hk_launch_gemm_few_rows_tile(dtype16, epi, a, i, n_tiles(a, kTiles[i]) <= 256, stream);
+}
+
+// The same with tile i of kTiles and its deep or shallow ring (tests reach every instance through it).
+extern "C" int hk_launch_gemm_few_rows_tile(int dtype16, int epi, const hk::GemmArgs* a, int i, int deep, hipStream_t stream) {
     if (a->M == 0) return HK_OK;
-    return dtype16 == hk::DT_BF16 ? launch_type<hk::bf16>(epi, a, stream) : launch_type<hk::f16>(epi, a, stream);
+    return dtype16 == hk::DT_BF16 ? launch_type<hk::bf16>(epi, a, i, deep, stream)
+                                  : launch_type<hk::f16>(epi, a, i, deep, stream);
 }

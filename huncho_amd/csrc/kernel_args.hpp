@@ -352,6 +352,7 @@ int hk_launch_gdn16_split(int dtype16, const hk::GdnArgs* a, const hk::GdnFusedA
 int hk_launch_gemm(int dtype16, int epi, const hk::GemmArgs* a, hipStream_t stream);
 float hk_gemm_few_rows_cost(int epi, const hk::GemmArgs* a);
 int hk_launch_gemm_few_rows(int dtype16, int epi, const hk::GemmArgs* a, hipStream_t stream);
+int hk_launch_gemm_few_rows_tile(int dtype16, int epi, const hk::GemmArgs* a, int i, int deep, hipStream_t stream);
 int hk_launch_lora_merge(int dtype, void* w, long rows, int cols, const float* a, const float* b, int rank, float scale,
                          hipStream_t st);
 int hk_launch_bidir_attention(int dtype, const hk::BertAttnArgs* a, int n_seqs, int max_len, hipStream_t stream);
