@@ -580,9 +580,9 @@ extern "C" int hk_kev_model_identity(hk_kev_model* m, char* buf, size_t len, siz
     const bool gdn_mfma = c.lin_key_dim == 128 && c.lin_v_dim == 128;
     const char* attn_exec = !attn_mfma ? "rocm-paged-general-wave-per-row-v1"
                             : f32      ? "rocm-paged-flash-mfma-f32-v1"
-                                       : "rocm-paged-flash-mfma-16bit-v1";
+                                       : "rocm-paged-flash-mfma-16bit-suffix-key-split-v2";
     const char* delta_exec = !gdn_mfma ? "rocm-recurrent-per-token-general-v1"
-                             : f32     ? "rocm-chunked-c64-mfma-f32-v1"
+                             : f32     ? "rocm-chunked-c64-mfma-f32-few-rows-split-v2"
                                        : "rocm-chunked-c64-mfma-f16-operands-v1";
     return hk_write_identity(
         {{"device", dev},

@@ -267,3 +267,18 @@ def test_identity_keys(ctx):
         seen[dt] = ident
     assert seen[torch.bfloat16]["activation_dtype"] == "bf16" and seen[torch.float16]["activation_dtype"] == "fp16"
     assert seen[torch.float32]["delta_rule_execution"] != seen[torch.bfloat16]["delta_rule_execution"]
+
+
+def test_identity_names_the_split_forms(ctx):
+    """Suffix attention and the fp32 delta rule of few rows add in another order than the kernels of large
+    batches, so the keys that name them are not those of a library without these forms. The 16-bit delta
+    rule's split form has the same bits, and its key stays."""
+    shape = KevShape(hidden=256, n_layers=4, n_heads=2, n_kv_heads=1, intermediate=512, vocab=1000,
+                     lin_n_k_heads=2, lin_n_v_heads=2, rotary_dim=64, n_out=3)
+    for dt, attn, delta in ((torch.bfloat16, "key-split", "rocm-chunked-c64-mfma-f16-operands-v1"),
+                            (torch.float16, "key-split", "rocm-chunked-c64-mfma-f16-operands-v1"),
+                            (torch.float32, "rocm-paged-flash-mfma-f32-v1", "few-rows-split")):
+        model = KevModel(ctx, shape, synthetic_weights(shape, 3), dt)
+        ident = abi.identity(abi.lib().hk_kev_model_identity, model.h)
+        model.close()
+        assert attn in ident["attention_execution"] and delta in ident["delta_rule_execution"]
