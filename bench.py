@@ -245,7 +245,7 @@ def fp32_config_kernels(ctx, iters):
     return {
         "attention_fp32_T256": entry("paged_prefill_attn_f32 (1 x 256, 16q/8kv x 128, P 16 identity table)",
                                      t_attn, attn_flops, attn_bytes),
-        "delta_rule_fp32_T512": entry("gdn_chunk_f32 (1 x 512, 16 x 128, chunk 64, final state)", t_gdn, rec_flops,
+        "delta_rule_fp32_T512": entry("delta_split_prep, _scan and _out (1 x 512, 16 x 128, chunk 64, final state)", t_gdn, rec_flops,
                                       gdn_bytes, {"chunked_tflops": round(chunk_flops / t_gdn / 1e12, 3)}),
     }
 

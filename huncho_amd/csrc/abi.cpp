@@ -772,8 +772,6 @@ extern "C" int hk_swiglu(hk_ctx* ctx, int dtype, const void* gu, long gu_tok, lo
     return rc ? hk_fail(ctx, rc, "swiglu launch failed") : HK_OK;
 }
 
-// The fused layer with optional per-sequence row tables for the state and the conv history
-// (device arrays of n_seqs pointers; used by the cached model forward).
 // Whether the batch takes the three-kernel form of the fused layer (gdn16_split.hip): few chains (pairs of
 // a row and a head), whose rows are several chunks long on average. Measured, 16 heads, bf16, us, one
 // kernel against three, by rows x tokens:
@@ -784,6 +782,8 @@ static bool gdn_split_takes(int n_seqs, int n_tokens, int heads) {
     return chains <= 64 ? chunks >= 2L * n_seqs : chains <= 128 && chunks >= 4L * n_seqs;
 }
 
+// The fused layer with optional per-sequence row tables for the state and the conv history
+// (device arrays of n_seqs pointers; used by the cached model forward).
 int hk_gdn_fused_rows(hk_ctx* ctx, int dtype, const void* mixed, long mixed_tok, const float* conv_w, int conv_k,
                       const void* conv_hist, void* conv_tail_out, const void* ba, long ba_tok, int b_col, int a_col,
                       const float* base_g, const float* dt_bias, const void* z, long z_tok, const float* norm_w,

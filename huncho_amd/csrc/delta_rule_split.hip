@@ -13,6 +13,7 @@
 //
 // Measured (16 heads, one row of 512 tokens with its final state): 268 -> 54 us, as far from the recurrence
 // in 64 bits as before (9.6e-7). delta_split_takes (abi.cpp) has the rule and the times on both sides of it.
+#include "chunk_slots.hpp"
 #include "delta_rule.hpp"
 
 namespace hk {
@@ -30,32 +31,9 @@ static_assert(SLOT * 4 == HK_DELTA_SPLIT_SLOT, "slot size in kernel_args.hpp");
 constexpr int WC = 16;                  // value columns per scan workgroup
 constexpr int SSTR = DK + 4, RSTR = CH + 4;
 
-__device__ __forceinline__ bool seq_rows(const GdnArgs& a, int s, int& t0, int& Tn) {
-    t0 = a.cu_seqlens[s];
-    Tn = a.cu_seqlens[s + 1] - t0;
-    return t0 >= 0 && Tn >= 0 && t0 + Tn <= a.n_tokens;
-}
-// Slots are numbered chunk by chunk, row by row; rows outside the batch have none.
-__device__ __forceinline__ int first_chunk(const GdnArgs& a, int s) {
-    int n = 0;
-    for (int i = 0; i < s; ++i) {
-        int t0, Tn;
-        if (seq_rows(a, i, t0, Tn)) n += (Tn + CH - 1) / CH;
-    }
-    return n;
-}
-__device__ __forceinline__ bool find_chunk(const GdnArgs& a, int n_seqs, int cid, int& c0, int& t0, int& Tn) {
-    for (int s = 0; s < n_seqs; ++s) {
-        if (!seq_rows(a, s, t0, Tn)) continue;
-        const int n = (Tn + CH - 1) / CH;
-        if (cid < n) {
-            c0 = cid * CH;
-            return true;
-        }
-        cid -= n;
-    }
-    return false;
-}
+using chunk_slots::find_chunk;
+using chunk_slots::first_chunk;
+using chunk_slots::seq_rows;
 
 __global__ __launch_bounds__(256, 1) void delta_split_prep(GdnArgs a, int n_seqs, float* scratch) {
     extern __shared__ __attribute__((aligned(16))) float smem_f[];
@@ -68,8 +46,8 @@ __global__ __launch_bounds__(256, 1) void delta_split_prep(GdnArgs a, int n_seqs
     float* Gs = Xs + 32 * XSTR;
     float* Bs = Gs + CH;
     const int h = blockIdx.x, cid = blockIdx.y;
-    int c0, t0, Tn;
-    if (!find_chunk(a, n_seqs, cid, c0, t0, Tn)) return;
+    int seq, c0, t0, Tn;
+    if (!find_chunk(a, n_seqs, cid, seq, c0, t0, Tn)) return;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     {
         const int t = t0 + c0, Lc = min(CH, Tn - c0);
@@ -243,8 +221,8 @@ __global__ __launch_bounds__(256, 2) void delta_split_out(GdnArgs a, int n_seqs,
     __shared__ __attribute__((aligned(16))) float Qs[CH * F_KSTR];
     __shared__ __attribute__((aligned(16))) float Aq[CH * F_ASTR];
     const int h = blockIdx.x, cid = blockIdx.y;
-    int c0, t0, Tn;
-    if (!find_chunk(a, n_seqs, cid, c0, t0, Tn)) return;
+    int seq, c0, t0, Tn;
+    if (!find_chunk(a, n_seqs, cid, seq, c0, t0, Tn)) return;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, q4 = lane >> 4, j = lane & 15;
     const int Lc = min(CH, Tn - c0), col = 64 * blockIdx.z + 16 * wave + j;
     const float* const slot = scratch + ((long)cid * a.H + h) * SLOT;

@@ -23,6 +23,7 @@
 //
 // Measured (bf16, 16 heads, one row of 2704 tokens with its state): prep 29, scan 44, out 15 us, the
 // whole 521 -> 94 us. gdn_split_takes (abi.cpp) has the rule and the times on both sides of it.
+#include "chunk_slots.hpp"
 #include "gdn16_kernel.hpp"
 
 namespace hk {
@@ -50,34 +51,9 @@ static_assert(STAGE % 1024 == 0 && COPIES <= 63, "vmcnt counts a stage of copies
 // The block (i, jj), jj <= i, of the lower triangle in the order the slots hold it
 __device__ __forceinline__ int tri(int i, int jj) { return i * (i + 1) / 2 + jj; }
 
-// The rows of sequence s: false (and a fault) if cu_seqlens is inconsistent there
-__device__ __forceinline__ bool seq_rows(const GdnArgs& a, int s, int& t0, int& Tn) {
-    t0 = a.cu_seqlens[s];
-    Tn = a.cu_seqlens[s + 1] - t0;
-    return t0 >= 0 && Tn >= 0 && t0 + Tn <= a.n_tokens;
-}
-// First slot number of sequence s (slots are numbered chunk by chunk, row by row; faulty rows have none)
-__device__ __forceinline__ int first_chunk(const GdnArgs& a, int s) {
-    int n = 0;
-    for (int i = 0; i < s; ++i) {
-        int t0, Tn;
-        if (seq_rows(a, i, t0, Tn)) n += (Tn + CH - 1) / CH;
-    }
-    return n;
-}
-// Chunk number cid -> sequence and first token of the chunk in it; false past the last chunk
-__device__ __forceinline__ bool find_chunk(const GdnArgs& a, int n_seqs, int cid, int& seq, int& c0, int& t0, int& Tn) {
-    for (seq = 0; seq < n_seqs; ++seq) {
-        if (!seq_rows(a, seq, t0, Tn)) continue;
-        const int n = (Tn + CH - 1) / CH;
-        if (cid < n) {
-            c0 = cid * CH;
-            return true;
-        }
-        cid -= n;
-    }
-    return false;
-}
+using chunk_slots::find_chunk;
+using chunk_slots::first_chunk;
+using chunk_slots::seq_rows;
 
 // P0 of gdn_chunk16 as a function: here the compiler does better with it (row of 2704 tokens, bf16, 1 % of the layer)
 template <typename T>
