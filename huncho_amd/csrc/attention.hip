@@ -107,7 +107,7 @@ __device__ __forceinline__ long part_index(const AttnArgs& a, int seq, int qb, i
 // weights applied to V sum to one.
 //
 // SPLIT: a batch of few rows leaves most CUs idle (five 30-token questions over one 2,700-token state:
-// 40 workgroups of 43 tiles, 54.9 us; split 13 and 6 for attn_combine). Then a workgroup takes one q-block and
+// 40 workgroups of 43 tiles, 54.9 us; split 17.4 and 4.7 for attn_combine). Then a workgroup takes one q-block and
 // one range of its key tiles, and writes its unnormalised fp32 O rows with their max and sum; attn_combine adds the ranges of a
 // row in their order. A q-block with a single range is finished here as in the unsplit kernel. A range
 // may lie past a row's last visible key: its max stays -inf and its probabilities 0.
