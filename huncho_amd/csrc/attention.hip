@@ -89,7 +89,7 @@ __device__ __forceinline__ int lds_off_k(int r, int c) { return r * KV_ROW + 8 *
 // range), and the first part of a q-block. A row is split by its own lengths, so that a row without cached
 // tokens is finished in one range whatever batch or table it comes with.
 __device__ __forceinline__ int split_range(const AttnArgs& a, int nt, int ctx, int q_len) {
-    if ((ctx + BN - 1) / BN < a.split_from || ctx / 4 < q_len) return nt;
+    if (ctx <= (a.split_from - 1) * BN || (ctx >> 2) < q_len) return nt;
     return nt <= 4 * a.n_split ? min(nt, 4) : (nt + a.n_split - 1) / a.n_split;
 }
 __device__ __forceinline__ long part_index(const AttnArgs& a, int seq, int qb, int kvh) {
@@ -132,6 +132,8 @@ __global__ __launch_bounds__(256, NH == 1 ? 2 : 1) void paged_prefill_attn_16(At
     const int kvh = blockIdx.x;
     const int z = SPLIT ? 0 : blockIdx.y;
     const int seq = SPLIT ? blockIdx.y : blockIdx.z;
+    // SPLIT: the q-block, counted from the last, and its range
+    const int zb = SPLIT && a.n_qblocks > 1 ? blockIdx.z / a.n_split : 0, zr = SPLIT ? blockIdx.z - zb * a.n_split : 0;
     const int q0 = a.cu_seqlens_q[seq];
     const int q_len = a.cu_seqlens_q[seq + 1] - q0;
     const int ctx = a.context_lens[seq];
@@ -143,9 +145,9 @@ __global__ __launch_bounds__(256, NH == 1 ? 2 : 1) void paged_prefill_attn_16(At
     }
     // this workgroup's q-blocks: the mirrored pair (nq - 1 - z, z), so every workgroup of a
     // sequence runs nq + 1 key tiles; the longer block goes first
-    const int nq = (q_len + P - 1) / P;
+    const int nq = SPLIT ? (q_len + P - 1) >> p_shift : (q_len + P - 1) / P;
     // (SPLIT: q-blocks past n_qblocks, rows longer than max_q_len, have no part)
-    const int qb_a = SPLIT ? a.n_qblocks - 1 - (int)(blockIdx.z / a.n_split) : nq - 1 - z, qb_b = z;
+    const int qb_a = SPLIT ? a.n_qblocks - 1 - zb : nq - 1 - z, qb_b = z;
     if (SPLIT ? qb_a >= nq : 2 * z >= nq) return;
     const int n_blocks = SPLIT || qb_a == qb_b ? 1 : 2;
     const int off = ctx - q_len;  // absolute position of the first new query
@@ -155,7 +157,7 @@ __global__ __launch_bounds__(256, NH == 1 ? 2 : 1) void paged_prefill_attn_16(At
     // SPLIT: tiles i0 .. nt_a - 1 of the block's
     const int nt_all = block_tiles(qb_a), range = SPLIT ? split_range(a, nt_all, ctx, q_len) : nt_all;
     const bool split = SPLIT && range < nt_all;
-    const int i0 = SPLIT ? (int)(blockIdx.z % a.n_split) * range : 0;
+    const int i0 = zr * range;
     if (SPLIT && i0 >= nt_all) return;
     const int nt_a = SPLIT ? min(nt_all, i0 + range) : nt_all;
     const int n_sched = nt_a + (n_blocks == 2 ? block_tiles(qb_b) : 0);
@@ -165,7 +167,7 @@ __global__ __launch_bounds__(256, NH == 1 ? 2 : 1) void paged_prefill_attn_16(At
     const int tid = threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63, g = lane >> 5, col = lane & 31;
     const int row = wave * 32 + col;  // this lane's query row: (head in group, position)
-    const int hg = row / P, p = row % P;
+    const int hg = SPLIT ? row >> p_shift : row / P, p = SPLIT ? row & (P - 1) : row % P;
     const int head = kvh * a.group + hg;
 
     // per-lane LDS offsets (elements): K rows of S^T (row perm_key(col), chunk 2 ks + g) and
@@ -449,7 +451,7 @@ __global__ __launch_bounds__(256, NH == 1 ? 2 : 1) void paged_prefill_attn_16(At
     if (SPLIT && split) {
         const float l_tot = l_run + __shfl_xor(l_run, 32);
         if (!q_valid) return;  // rows past the sequence have no part (short suffixes fill half a block)
-        const long w = part_index(a, seq, qb_a, kvh) + blockIdx.z % a.n_split;
+        const long w = part_index(a, seq, qb_a, kvh) + zr;
         float* const op = a.part + (w * 128 + row) * HD + 4 * g;
 #pragma unroll
         for (int db = 0; db < 4 * NH; ++db)
@@ -484,10 +486,10 @@ __global__ __launch_bounds__(256) void attn_combine(AttnArgs a) {
     if (q0 < 0 || q_len < 0 || q0 + q_len > a.n_tokens || q_len > ctx || qb * P >= q_len) return;
     const int nt = (ctx - q_len + min(q_len, (qb + 1) * P) - 1) / BN + 1, range = split_range(a, nt, ctx, q_len);
     if (range >= nt) return;  // finished by the attention kernel
-    const int ns = (nt + range - 1) / range;
+    const int ns = range == 4 ? (nt + 3) / 4 : (nt + range - 1) / range;
     const long w0 = part_index(a, seq, qb, kvh);
     const int row = RPP * (blockIdx.y % (128 / RPP)) + threadIdx.x / LPR, d = 4 * (threadIdx.x % LPR);
-    const int qi = qb * P + (row & (P - 1)), head = kvh * a.group + row / P;
+    const int qi = qb * P + (row & (P - 1)), head = kvh * a.group + (row >> __builtin_ctz(P));
     if (qi >= q_len) return;  // the same for a row's lanes
     // lane i of each 32 holds range i's max and sum: one load, then the weights by shuffle
     const int i = threadIdx.x & 31;
