@@ -228,8 +228,9 @@ static float library_us(const hk::GemmArgs& a) {
 // 13.8, at 512 rows 17.0 and 14.8, at 600 (library) 22 and 16.4; 1024 x 3584 + residual at 300 rows 12.3 against
 // 17.2, at 1024 (library) 19.6 and 18.9, at 4096 (library) 46.1 and 36.6; 768 x 1152 + residual at 1700 rows 9.8 against
 // 10.6, at 2704 (library) 14.6 and 12.7; 32 x 1024 at 16384 rows 5.4 against 10.1, at 32768 (library) 11.7 and 13.2.
-// The few-row kernel's sums do not depend on the number of rows. The library's choice for some small batches
-// adds in another order, and there the two differ by the rounding of their sums.
+// The few-row kernel's sums do not depend on the number of rows. The library's choice for the smallest batches
+// adds in another order, and there the two differ by the rounding of their sums: up to 16 rows of 2304 to 8192
+// columns, 31 of 768 x 768, 127 of 1024 columns + residual, and up to 160 and around 330 of 768 x 1152.
 static bool few_rows_wins(int epi, const hk::GemmArgs& a) { return few_rows_us(epi, a) <= 0.93f * library_us(a); }
 // The way such a projection takes, estimated
 static float projection_us(const hk::GemmArgs& a) {

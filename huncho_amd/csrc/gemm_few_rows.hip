@@ -10,8 +10,8 @@
 // Each output is one chain of fp32 accumulations over K in order, whatever the tile or the number of
 // rows, so a row's result does not change with the batch it comes in: SwiGLU on the 32x32x16 products
 // of gemm.hip (the same bits as that kernel), store and residual on 16x16x32 products (the same bits as
-// the library's kernels of the large batches, so a prefix computed alone agrees with whole rows in a batch; for some
-// small batches the library's choice adds in another order, which the sums here replaced).
+// the library's kernels of the large batches, so a prefix computed alone agrees with whole rows in a batch; for the
+// smallest batches, few_rows_wins in blas.cpp, the library's choice added in another order).
 // (A split of K over the four waves, each with a ring of its own, ran as fast but gave other sums.)
 //
 // Measured (us, bf16, weights rotated through 600 MB so that they come from HBM; gemm.hip beside it):
